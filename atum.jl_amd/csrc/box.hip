@@ -1,0 +1,228 @@
+// Box elements: detection from an operator's geometry arrays (box.hpp).
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstring>
+
+#include "box.hpp"
+#include "handles.hpp"
+
+namespace {
+
+// The record of direction count `dim` at `rec`, written field by field (BoxElem<dim>'s layout)
+__device__ void store_record(char* rec, int dim, const double* g, double J, const double* fJ, const int32_t* nb) {
+  double* d = reinterpret_cast<double*>(rec);
+  for (int r = 0; r < dim; ++r) d[r] = g[r];
+  d[dim] = J;
+  for (int r = 0; r < dim; ++r) d[dim + 1 + r] = fJ[r];
+  int32_t* n = reinterpret_cast<int32_t*>(d + 2 * dim + 1);
+  for (int f = 0; f < 2 * dim; ++f) n[f] = nb[f];
+}
+
+constexpr int CAND = 5;  // Jacobians tried: the quotient of the first entry and its weight, and 2 ulps either side
+
+__device__ double candidate(double x, int c) {
+  return __longlong_as_double(__double_as_longlong(x) + (c - CAND / 2));
+}
+
+// the candidate to keep: the quotient itself if it fits, else any that does
+__device__ int pick(unsigned mask) { return (mask >> (CAND / 2)) & 1u ? CAND / 2 : __ffs(mask) - 1; }
+
+// One workgroup per element: writes its record, or sets *bad when its arrays are not those of a box.
+__global__ void __launch_bounds__(256)
+    box_detect_kernel(DevDG p, int dim, const double* __restrict__ wp, const double* __restrict__ wf, char* rec,
+                      int bytes, int32_t* bad) {
+  __shared__ unsigned mJ, mF[3];
+  __shared__ int ok;
+  for (int64_t e = blockIdx.x; e < p.K; e += gridDim.x) {
+    if (threadIdx.x == 0) {
+      mJ = mF[0] = mF[1] = mF[2] = (1u << CAND) - 1;
+      ok = 1;
+    }
+    __syncthreads();
+    bool good = true;
+    const double J0 = p.MJ[e * p.Np] / wp[0];
+    good = good && J0 > 1e-300 && J0 < 1e300;
+    unsigned m = (1u << CAND) - 1;
+    for (int t = threadIdx.x; t < p.Np; t += blockDim.x) {
+      const int64_t node = e * p.Np + t;
+      const double mj = p.MJ[node];
+      for (int c = 0; c < CAND; ++c)
+        if (wp[t] * candidate(J0, c) != mj) m &= ~(1u << c);
+      good = good && 1 / mj == p.MJI[node];
+      for (int a = 0; a < dim; ++a)
+        for (int c = 0; c < dim; ++c) {
+          const int64_t at = (int64_t)(a + dim * c) * p.Ntot;
+          good = good && p.g[at + node] == (a == c ? p.g[at + e * p.Np] : 0.0);
+        }
+    }
+    atomicAnd(&mJ, m);
+    double fJ0[3] = {1, 1, 1};
+    unsigned mf[3] = {(1u << CAND) - 1, (1u << CAND) - 1, (1u << CAND) - 1};
+    for (int r = 0; r < dim; ++r) {
+      fJ0[r] = p.faceMJ[e * p.Nfp + 2 * r * p.Nfpf] / wf[0];
+      good = good && fJ0[r] > 1e-300 && fJ0[r] < 1e300;
+    }
+    for (int f = threadIdx.x; f < p.Nfp; f += blockDim.x) {
+      const int face = f / p.Nfpf, fp = f - face * p.Nfpf, r = face >> 1, side = face & 1;
+      const int64_t jj = e * p.Nfp + f;
+      for (int c = 0; c < CAND; ++c)
+        if (wf[fp] * candidate(fJ0[r], c) != p.faceMJ[jj]) mf[r] &= ~(1u << c);
+      for (int d = 0; d < dim; ++d)
+        good = good && p.normal[d * p.NF + jj] == (d == r ? (side ? 1.0 : -1.0) : 0.0);
+      if (p.bctag[e * (2 * dim) + face] == 0) {
+        // the same point of the opposite face of one element
+        int st = 1, pos = 0, rem = fp;
+        for (int d = 0; d < dim; ++d) {
+          if (d == r) {
+            pos += (side ? 0 : p.Nq - 1) * st;
+          } else {
+            pos += (rem % p.Nq) * st;
+            rem /= p.Nq;
+          }
+          st *= p.Nq;
+        }
+        const int64_t en = p.faceix_p[e * p.Nfp + face * p.Nfpf] / p.Np;
+        good = good && p.faceix_p[jj] == en * p.Np + pos;
+      }
+    }
+    for (int r = 0; r < dim; ++r) atomicAnd(&mF[r], mf[r]);
+    if (!good) ok = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      bool box = ok && mJ;
+      for (int r = 0; r < dim; ++r) box = box && mF[r];
+      if (box) {
+        double g[3], fJ[3];
+        int32_t nb[6];
+        for (int r = 0; r < dim; ++r) {
+          g[r] = p.g[(int64_t)(r + dim * r) * p.Ntot + e * p.Np];
+          fJ[r] = candidate(fJ0[r], pick(mF[r]));
+        }
+        for (int f = 0; f < 2 * dim; ++f) {
+          const int tag = p.bctag[e * (2 * dim) + f];
+          nb[f] = tag ? -tag : (int32_t)(p.faceix_p[e * p.Nfp + f * p.Nfpf] / p.Np);
+        }
+        store_record(rec + e * bytes, dim, g, candidate(J0, pick(mJ)), fJ, nb);
+      } else {
+        *bad = 1;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// LGL weights 2 / (N (N+1) P_N(x)^2), the nodes by Newton on P_N' in extended precision
+void lgl_weights(int Nq, double* w) {
+  const int N = Nq - 1;
+  auto legendre = [](int n, long double x) {
+    long double a = 1, b = x;
+    if (n == 0) return a;
+    for (int k = 2; k <= n; ++k) {
+      const long double c = ((2 * k - 1) * x * b - (k - 1) * a) / k;
+      a = b;
+      b = c;
+    }
+    return b;
+  };
+  for (int i = 0; i < Nq; ++i) {
+    long double P = 1;
+    if (i > 0 && i < N) {
+      long double x = -std::cos(3.14159265358979323846L * i / N);
+      for (int it = 0; it < 30; ++it) {
+        const long double p0 = legendre(N, x), p1 = legendre(N - 1, x);
+        const long double dP = N * (p1 - x * p0) / (1 - x * x);
+        const long double d2P = (2 * x * dP - N * (N + 1) * p0) / (1 - x * x);
+        x -= dP / d2P;
+      }
+      P = legendre(N, x);
+    }
+    w[i] = (double)(2 / (N * (N + 1) * P * P));
+  }
+}
+
+}  // namespace
+
+namespace atm {
+
+int dg_box(atm_dg* dg, const atm_dg_desc* d, const double* w_host) {
+  DevDG& p = dg->dev;
+  if (p.K < 1) return ATM_OK;
+  const Resolved r = resolve_box(d, dg->Nq);
+  atm_ctx* ctx = dg->ctx;
+  if (!r.fn || r.lds > ctx->max_lds) return ATM_OK;
+  const int dim = dg->dim, Nq = dg->Nq, Np = dg->Np;
+  std::vector<double> tab((size_t)Nq + Np + p.Nfpf);
+  double* w = tab.data();
+  double* wp = w + Nq;
+  double* wf = wp + Np;
+  if (w_host) std::memcpy(w, w_host, sizeof(double) * Nq);
+  else lgl_weights(Nq, w);
+  for (int t = 0; t < Np + p.Nfpf; ++t) {
+    int rem = t < Np ? t : t - Np;
+    double v = 1.0;
+    for (int i = 0; i < (t < Np ? dim : dim - 1); ++i) {
+      v = v * w[rem % Nq];
+      rem /= Nq;
+    }
+    (t < Np ? wp[t] : wf[t - Np]) = v;
+  }
+  const size_t bytes = (size_t)(2 * dim + 1) * sizeof(double) + (size_t)2 * dim * sizeof(int32_t);
+  const size_t head = (tab.size() * sizeof(double) + sizeof(int32_t) + 255) / 256 * 256;
+  void* mem = nullptr;
+  HIPCHK(ctx, hipMalloc(&mem, head + bytes * (size_t)p.K));
+  double* dtab = static_cast<double*>(mem);
+  int32_t* bad = reinterpret_cast<int32_t*>(dtab + tab.size());
+  char* rec = static_cast<char*>(mem) + head;
+  std::vector<char> init(tab.size() * sizeof(double) + sizeof(int32_t), 0);  // weights, then the flag
+  std::memcpy(init.data(), tab.data(), tab.size() * sizeof(double));
+  hipStream_t s = stream_of(ctx);
+  int32_t host_bad = 1;
+  hipError_t e = hipMemcpy(mem, init.data(), init.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(box_detect_kernel, dim3(p.K < 65536 ? p.K : 65536), dim3(256), 0, s, p, dim, dtab + Nq,
+                       dtab + Nq + Np, rec, (int)bytes, bad);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = hipMemcpy(&host_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost);
+  if (e != hipSuccess || host_bad) {
+    hipFree(mem);
+    return e == hipSuccess ? ATM_OK : hipfail(ctx, e, "box element detection");
+  }
+  dg->allocs.push_back(mem);
+  dg->dev_bytes += head + bytes * (size_t)p.K;
+  p.box = rec;
+  p.bw = dtab;
+  dg->fn = r.fn;
+  dg->bfn = r.bfn;
+  dg->mbfn = r.mbfn;
+  dg->lds = r.lds;
+  dg->epw = r.epw;
+  dg->lds_fixed = r.lds_fixed;
+  dg->lds_elem = r.lds_elem;
+  dg->max_threads = r.max_threads;
+  p.epw = r.epw;
+  p.lds = (int)r.lds;
+  return ATM_OK;
+}
+
+Resolved resolve_box_weak_euler(int dim, int mask, int Nq);
+Resolved resolve_box_weak_euler_gravity(int dim, int mask, int Nq);
+Resolved resolve_box_weak_linear(int dim, int mask, int Nq);
+Resolved resolve_box_weak_shallow_water(int dim, int mask, int Nq);
+
+// Kernels for an operator whose elements are all boxes (fn == nullptr: the general ones)
+Resolved resolve_box(const atm_dg_desc* d, int Nq) {
+  if (d->volume_form == ATM_FORM_WEAK && d->surface_flux == ATM_FLUX_RUSANOV) switch (d->law) {
+      case ATM_LAW_ADVECTION: return weak_box_dims<Advection, ATM_FLUX_RUSANOV, true>(d->dim, d->dirmask, Nq);
+      case ATM_LAW_EULER: return resolve_box_weak_euler(d->dim, d->dirmask, Nq);
+      case ATM_LAW_EULER_GRAVITY: return resolve_box_weak_euler_gravity(d->dim, d->dirmask, Nq);
+      case ATM_LAW_LINEAR_EULER_GRAVITY: return resolve_box_weak_linear(d->dim, d->dirmask, Nq);
+      case ATM_LAW_SHALLOW_WATER: return resolve_box_weak_shallow_water(d->dim, d->dirmask, Nq);
+      default: break;
+    }
+  return Resolved{nullptr, 0, 0, nullptr, 1};
+}
+
+}  // namespace atm

@@ -1,0 +1,325 @@
+// Box elements: the compact geometry of axis-aligned rectangular elements.
+//
+// Every element of a brick mesh is an axis-aligned box: its metric is the diagonal 2/h in
+// every node, MJ and faceMJ are the element's Jacobians times products of the LGL weights,
+// its normals are the unit vectors and a face's neighbour nodes are the opposite face of one
+// element in the same order.  The element kernels of such an operator read one BoxElem per
+// element instead of d^2 + 2 doubles per node and d + 2 per face point: for 2-D N = 3 that is
+// 56 bytes per element of 16 nodes instead of 1280 (the state, dq and the new state are 2048).
+//
+// Whether an operator's elements are boxes is found from its geometry arrays when it is
+// created (box_detect): the values that the compact form reproduces have to equal the arrays
+// bit for bit in every node and face point, so that both forms of a kernel compute with the
+// same numbers.  Operators with any other element keep the general kernels.
+#pragma once
+#include <type_traits>
+
+#include "dg_kernels.hpp"
+
+namespace atm {
+
+template <int D>
+struct BoxElem {
+  double g[D];        // 2/h: the diagonal of the metric
+  double J;           // MJ = wp * J, wp the product of the node's LGL weights; MJI = 1/MJ
+  double fJ[D];       // faceMJ = wf * fJ[r] on the faces of direction r
+  int32_t nb[2 * D];  // neighbour element of each face, or minus the boundary tag
+};
+
+template <int D>
+ATM_DEV const BoxElem<D>& box_elem(const DevDG& p, int64_t e) {
+  return static_cast<const BoxElem<D>*>(p.box)[e];
+}
+
+constexpr int ipow(int b, int n) { return n == 0 ? 1 : b * ipow(b, n - 1); }
+
+// The direction mask of an operator of all directions
+template <class L>
+constexpr int all_dirs() {
+  return (1 << L::D) - 1;
+}
+
+// Line stride of direction R in an element's node numbering
+template <int NQ, int R>
+constexpr int line_stride() {
+  return ipow(NQ, R);
+}
+
+// Compile-time loop over the directions
+template <int R, int D, class F>
+ATM_DEV void for_dirs(F&& f) {
+  if constexpr (R < D) {
+    f(std::integral_constant<int, R>{});
+    for_dirs<R + 1, D>(f);
+  }
+}
+
+// Wave speed with the unit normal of direction R (the laws' wavespeed with the other
+// components of the normal zero)
+template <class L, int R>
+ATM_DEV double axis_wavespeed(const LawConst& c, const double* q, const double* a) {
+  constexpr int D = L::D;
+  if constexpr (L::LAW == ATM_LAW_ADVECTION) {
+    return fabs(c.u[R]);
+  } else if constexpr (L::LAW == ATM_LAW_LINEAR_EULER_GRAVITY) {
+    return L::wavespeed(c, nullptr, q, a);
+  } else if constexpr (L::LAW == ATM_LAW_SHALLOW_WATER) {
+    return fabs(q[1 + R] / q[0]) + sqrt(c.grav * q[0]);
+  } else {
+    double p;
+    if constexpr (L::LAW == ATM_LAW_EULER_GRAVITY) p = L::pressure(c, q[0], q + 1, q[D + 1], a[0]);
+    else p = L::pressure(c, q[0], q + 1, q[D + 1]);
+    return fabs(q[1 + R] / q[0]) + sqrt(c.gamma * p / q[0]);
+  }
+}
+
+// surfaceflux<L, SF> with the normal sg * e_R, sg = +-1: the products with the normal's zeros
+// and ones are left out, so the result is the same value (up to the sign of a zero)
+template <class L, int SF, int R>
+ATM_DEV void axis_surfaceflux(const LawConst& c, double sg, const double* qm, const double* am, const double* qp,
+                              const double* ap, double* nf) {
+  constexpr int D = L::D, Ns = L::Ns;
+  if constexpr (SF == ATM_FLUX_ROE || SF == ATM_FLUX_MATRIX) {
+    double n[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) n[d] = d == R ? sg : 0.0;
+    L::template special_surface<SF>(c, n, qm, am, qp, ap, nf);
+  } else {
+    double F[D][Ns];
+    constexpr int TP = (SF == ATM_FLUX_RUSANOV) ? ATM_FLUX_CENTRAL : SF;
+    L::template twopoint<TP>(c, qm, am, qp, ap, F);
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) nf[s] = sg * F[R][s];
+    if constexpr (SF == ATM_FLUX_RUSANOV) {
+      const double ws = fmax(axis_wavespeed<L, R>(c, qm, am), axis_wavespeed<L, R>(c, qp, ap));
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) nf[s] = nf[s] - ws * (qp[s] - qm[s]) / 2;
+    }
+  }
+}
+
+// Surface contributions of the faces this node lies on, subtracted from acc (surface_node on
+// box elements).  sw: the LGL weights.
+template <class L, int SF, int NQ, int MASK>
+ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, int64_t e, int ijk, const int idx[3],
+                              const double* q, const double* qn, const double* an, double MJIn, const double* sw,
+                              double* acc) {
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D);
+  for_dirs<0, D>([&](auto R) {
+    constexpr int r = decltype(R)::value;
+    if constexpr (((MASK >> r) & 1) == 0) return;
+    const int ir = idx[r];
+    if (ir != 0 && ir != NQ - 1) return;
+    const bool hi = ir != 0;
+    const int nb = hi ? b.nb[2 * r + 1] : b.nb[2 * r];
+    constexpr int span = (NQ - 1) * line_stride<NQ, r>();
+    // a boundary node reads its own state as the neighbour's and replaces it by the boundary state
+    const int64_t idp = nb >= 0 ? (int64_t)nb * Np + ijk + (hi ? -span : span) : e * Np + ijk;
+    double qp[Ns], ap[NA], nf[Ns];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) qp[s] = q[s * p.Ntot + idp];
+    load_aux<L>(p, idp, ap);
+    const double sg = hi ? 1.0 : -1.0;
+    if (nb < 0) {
+      double n[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) n[d] = d == r ? sg : 0.0;
+      boundarystate<L>(p.c, n, qn, -nb, qp);
+#pragma unroll
+      for (int s = 0; s < NA; ++s) ap[s] = an[s];
+    }
+    axis_surfaceflux<L, SF, r>(p.c, sg, qn, an, qp, ap, nf);
+    double wf = 1.0;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (d != r) wf = wf * sw[idx[d]];
+    const double fMJ = wf * b.fJ[r];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) acc[s] -= fMJ * nf[s] * MJIn;
+  });
+}
+
+// ---------------------------------------------------------------------------
+// Weak form on box elements: weak_body with the compact geometry, the same operations in the
+// same order.  Only the flux row of a direction enters its sum (the metric is diagonal), and
+// LDS holds only the directions of the operator (the bits of MASK, fixed at compile time).
+// Bound by memory traffic.  Against the general kernels, per fused stage: 2-D shallow water, 256^2
+// elements, N = 3: 42.1 -> 28.4 us (134 MB of states: 4.7 TB/s); 3-D Euler, 20^3, N = 4, which had run
+// the runtime-degree kernel: 93.0 -> 49.4 us; 2-D advection, 80^2, N = 4: 6.6 -> 4.7 us.
+template <class L, int NQ, int SF, int MASK>
+ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
+                           double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
+                           int epw) {
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D);
+  double* sD = lds;
+  double* sw = lds + NQ * NQ;
+  constexpr int dirs = __builtin_popcount(MASK);
+  const int tid = threadIdx.x;
+  const int el = tid / Np;
+  const int ijk = tid - el * Np;
+  const int64_t le = blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < p.K;
+  const int64_t e = (p.sched && active) ? (int64_t)p.sched[le] : le;
+  double* slF = lds + NQ * NQ + NQ + el * (dirs * Ns * Np);  // [dir slot][s][node]
+  for (int t = tid; t < NQ * NQ; t += blockDim.x) sD[t] = p.D[t];
+  for (int t = tid; t < NQ; t += blockDim.x) sw[t] = p.bw[t];
+  double q1[Ns], a1[NA];
+  const int64_t el_e = active ? e : 0;  // a lane past the last element reads element 0 and discards it
+  const int64_t node = el_e * Np + ijk;
+  int idx[3];
+  node_index<D>(ijk, NQ, idx);
+  // every load first and unconditionally: the element's record, state, aux and the stage's dq in flight together
+  const BoxElem<D> b = box_elem<D>(p, el_e);
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) q1[s] = q[s * p.Ntot + node];
+  load_aux<L>(p, node, a1);
+  const double wp = p.bw[NQ + ijk];
+  double dq0[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) dq0[s] = 0.0;
+  if (!assign) {  // uniform over the launch
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) dq0[s] = dq[s * p.Ntot + node];
+  }
+  const double MJn = wp * b.J;
+  if (active) {
+    double F[D][Ns];
+    L::flux(p.c, q1, a1, F);
+    int slot = 0;
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+      if (!((MASK >> r) & 1)) continue;
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) slF[(slot * Ns + s) * Np + ijk] = b.g[r] * F[r][s] * MJn;
+      ++slot;
+    }
+  }
+  __syncthreads();
+  if (!active) return;
+  const double MJIn = 1 / MJn;
+  double dl[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) dl[s] = -0.0;
+  L::sources(p.c, dl, q1, a1, MASK, true);
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    double Dn[D];
+#pragma unroll
+    for (int r = 0; r < D; ++r) Dn[r] = sD[n + NQ * idx[r]] * MJIn;
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) {
+      int slot = 0;
+      int st = 1;
+#pragma unroll
+      for (int r = 0; r < D; ++r) {
+        if ((MASK >> r) & 1) {
+          dl[s] += Dn[r] * slF[(slot * Ns + s) * Np + ijk + (n - idx[r]) * st];
+          ++slot;
+        }
+        st *= NQ;
+      }
+    }
+  }
+  double acc[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) acc[s] = assign ? dl[s] : alpha * dq0[s] + dl[s];
+  box_surface_node<L, SF, NQ, MASK>(p, b, e, ijk, idx, q, q1, a1, MJIn, sw, acc);
+  epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+}
+
+ATM_KERNEL_PAIR(weak_box_kernel, weak_box_body, class L ATM_COMMA int NQ ATM_COMMA int SF ATM_COMMA int MASK,
+                L ATM_COMMA NQ ATM_COMMA SF ATM_COMMA MASK)
+
+// One launch per stage for members of different degrees (as weak_multi_kernel_batch)
+template <class L, int SF>
+__global__ void __launch_bounds__(512)
+    weak_box_multi_kernel_batch(const BatchEntry* __restrict__ tab, int n, int parity, double alpha, int assign,
+                                double b) {
+  extern __shared__ double lds[];
+  constexpr int M = all_dirs<L>();
+  const int64_t lb = xcd_block();
+  const int i = batch_find(tab, n, lb);
+  const DevDG p = tab[i].p;
+  const int64_t blk = lb - tab[i].block_start;
+  const double* qin = tab[i].buf[parity];
+  double* qo = tab[i].buf[1 - parity];
+  const double bdt = b * tab[i].dt;
+  switch (p.Nq) {
+    case 4: weak_box_body<L, 4, SF, M>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 5: weak_box_body<L, 5, SF, M>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 6: weak_box_body<L, 6, SF, M>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 7: weak_box_body<L, 7, SF, M>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 8: weak_box_body<L, 8, SF, M>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    default: break;
+  }
+}
+
+template <class L, int SF>
+hipError_t launch_weak_box_multi_batch(const BatchEntry* tab, int n, int64_t blocks, int threads, size_t lds, int epw,
+                                       hipStream_t st, int parity, double alpha, int assign, double b) {
+  (void)epw;  // every member carries its own in the table
+  hipLaunchKernelGGL((weak_box_multi_kernel_batch<L, SF>), dim3(blocks), dim3(threads), lds, st, tab, n, parity,
+                     alpha, assign, b);
+  return hipGetLastError();
+}
+
+template <class L, int NQ, int SF, int MASK>
+hipError_t launch_weak_box(const DevDG& p, hipStream_t st, const double* q, double* dq, double alpha, int assign,
+                           double* qout, double bdt) {
+  const int threads = ((p.epw * p.Np + 63) / 64) * 64;
+  if (p.epw < 1 || threads > 512) return hipErrorInvalidConfiguration;
+  const int blocks = (p.K + p.epw - 1) / p.epw;
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL((weak_box_kernel<L, NQ, SF, MASK>), dim3(blocks), dim3(threads), p.lds, st, p, q, dq, alpha, assign,
+                     qout, bdt, p.epw);
+  return hipGetLastError();
+}
+
+template <class L, int NQ, int SF, int MASK>
+hipError_t launch_weak_box_batch(const BatchEntry* tab, int n, int64_t blocks, int threads, size_t lds, int epw,
+                                 hipStream_t st, int parity, double alpha, int assign, double b) {
+  hipLaunchKernelGGL((weak_box_kernel_batch<L, NQ, SF, MASK>), dim3(blocks), dim3(threads), lds, st, tab, n, parity, alpha,
+                     assign, b, epw);
+  return hipGetLastError();
+}
+
+template <class L, int NQ, int SF, int MASK>
+Resolved make_weak_box() {
+  constexpr int Np = ipow(NQ, L::D);
+  return make_resolved(launch_weak_box<L, NQ, SF, MASK>, launch_weak_box_batch<L, NQ, SF, MASK>, L::Ns,
+                       elements_per_workgroup(Np), sizeof(double) * (NQ * NQ + NQ),
+                       sizeof(double) * __builtin_popcount(MASK) * L::Ns * Np);
+}
+
+template <class L, int SF, int MASK>
+Resolved weak_box_nq(int Nq) {
+  switch (Nq) {
+    case 2: return make_weak_box<L, 2, SF, MASK>();
+    case 3: return make_weak_box<L, 3, SF, MASK>();
+    case 4: return make_weak_box<L, 4, SF, MASK>();
+    case 5: return make_weak_box<L, 5, SF, MASK>();
+    case 6: return make_weak_box<L, 6, SF, MASK>();
+    case 7: return make_weak_box<L, 7, SF, MASK>();
+    case 8: return make_weak_box<L, 8, SF, MASK>();
+    default: return Resolved{nullptr, 0, 0, nullptr, 1};
+  }
+}
+
+// VERT: with the kernels of operators of the last direction only (the implicit half of an IMEX
+// pair) beside those of all directions; any other subset runs the general kernels
+template <class L, int SF, bool VERT>
+Resolved weak_box_mask(int mask, int Nq) {
+  if (mask == all_dirs<L>()) return weak_box_nq<L, SF, all_dirs<L>()>(Nq);
+  if constexpr (VERT && L::D > 1)
+    if (mask == 1 << (L::D - 1)) return weak_box_nq<L, SF, 1 << (L::D - 1)>(Nq);
+  return Resolved{nullptr, 0, 0, nullptr, 1};
+}
+
+template <template <int> class LAW, int SF, bool VERT>
+Resolved weak_box_dims(int dim, int mask, int Nq) {
+  if (dim == 1) return weak_box_mask<LAW<1>, SF, VERT>(mask, Nq);
+  if (dim == 2) return weak_box_mask<LAW<2>, SF, VERT>(mask, Nq);
+  return weak_box_mask<LAW<3>, SF, VERT>(mask, Nq);
+}
+
+}  // namespace atm

@@ -211,6 +211,10 @@ int atm_dg_create_brick(atm_ctx* ctx, const atm_dg_desc* d, const atm_brick_desc
   p.normal = (const double*)nrm;
   p.faceix_p = (const int64_t*)fxp;
   p.bctag = (const int32_t*)tag;
+  if ((rc = dg_box(dg, d, bd->w))) {
+    atm_dg_destroy(dg);
+    return rc;
+  }
   *out = dg;
   return ATM_OK;
 }

@@ -34,6 +34,10 @@ struct DevDG {
   const double* aux;
   const int64_t* faceix_p;
   const int32_t* bctag;
+  // box elements (box.hpp): one record per element, the LGL weights and their products; null
+  // for operators with any other element
+  const void* box;
+  const double* bw;  // weights (Nq), their products per node (Np) and face point (Nfpf)
 };
 
 // aux components the two-point fluxes read from neighbour nodes: Φ, ρ_ref, p_ref

@@ -89,6 +89,14 @@ inline int hipfail(atm_ctx* ctx, hipError_t e, const char* what) {
 // aux and boundary-state pointers still null).
 int dg_prepare(atm_ctx* ctx, const atm_dg_desc* d, atm_dg** out);
 
+// The kernels for an operator whose elements are all boxes (box.hpp); fn == nullptr if none.
+Resolved resolve_box(const atm_dg_desc* d, int Nq);
+
+// Looks whether the operator's elements are all boxes, its geometry arrays being on the device;
+// if so, and there are kernels for it, builds the compact geometry and selects them.  w_host: the LGL
+// weights the geometry was built with (null: computed here).
+int dg_box(atm_dg* dg, const atm_dg_desc* d, const double* w_host);
+
 // The linear operator a banded factorisation was built from.
 atm_dg* banded_lin(const atm_banded* b);
 

@@ -1,0 +1,104 @@
+"""Box elements: operators whose elements are all axis-aligned boxes run kernels on a compact
+geometry; any other element keeps the general ones.  The general kernels are reached here with the
+last node's MJI one ulp off, which is no box's, so both forms compute on otherwise equal geometry."""
+import numpy as np
+import pytest
+
+import problems as P
+from gpu_cases import _flux, make_state
+
+pytestmark = pytest.mark.gpu
+
+
+def pair(law, dim, N, Kd, form="weak", sflux="rusanov", bc="copy", periodic=True, directions=None,
+         ordering="cartesian", precision="reference", source=None, seed=0, geometry="host", level=False):
+    """(box operator, general operator, state); uneven coordinates, so that every box differs."""
+    import atum_hip as A
+    rng = np.random.default_rng(seed)
+    size = 2000.0 if "gravity" in law else 2.0
+    coords = [np.concatenate([[0.0], np.cumsum(rng.uniform(0.7, 1.3, k))]) * size / k for k in Kd]
+    per = (periodic,) * dim if isinstance(periodic, bool) else periodic
+    prob = A.Problem(boundary=bc, source=source, omega=1e-2,
+                     bc_states=rng.uniform(1, 2, (2 * dim, dim + 2)) if bc == "prescribed" else None)
+    u = (1.0, -0.4, 0.7)[:dim]
+
+    def build(off):
+        g = A.brickgrid(A.LobattoCell(N, dim), coords, per, ordering)
+        if off:
+            g.MJI = g.MJI.copy()
+            g.MJI[-1] = np.nextafter(g.MJI[-1], np.inf)
+        if law == "advection":
+            alaw = A.AdvectionLaw(dim, u, problem=prob)
+        elif law == "euler":
+            alaw = A.EulerLaw(dim, problem=prob)
+        elif law == "shallow_water":
+            alaw = A.ShallowWaterLaw(dim, grav=9.81, problem=prob)
+        else:
+            prob.referencestate = lambda x: P.isothermal_reference(x)
+            alaw = A.EulerGravityLaw(dim, problem=prob, pde_level_balance=level)
+            if law == "linear_euler_gravity":
+                alaw = A.LinearEulerGravityLaw(alaw)
+        vf = A.WeakForm() if form == "weak" else A.FluxDifferencingForm(_flux(A, form))
+        return A.DGSEM(law=alaw, grid=g, volume_form=vf, surface_numericalflux=_flux(A, sflux),
+                       directions=directions, precision=precision, geometry="host" if off else geometry)
+
+    box, general = build(False), build(True)
+    q = make_state(law, box.grid.points, rng, box.auxstate)
+    if "gravity" in law and law != "linear_euler_gravity":
+        q = make_state("euler_gravity", box.grid.points, rng, box.auxstate)
+    return box, general, q
+
+
+def device_bytes(dg):
+    import atum_hip._lib as L
+    return L.lib.atm_dg_device_bytes(dg.h)
+
+
+def tendencies(box, general, q0):
+    out = []
+    for dg in (box, general):
+        q = dg.fieldarray(q0)
+        dq = dg.fieldarray(np.cos(np.arange(q0.size)).reshape(q0.shape))
+        dg(dq, q, 0.0, increment=True)
+        dg.ctx.sync()
+        out.append(dq.numpy())
+    return out
+
+
+WEAK = [("advection", 1, (7,), {}), ("advection", 2, (5, 3), dict(bc="zero_inflow", periodic=(True, False))),
+        ("advection", 3, (3, 2, 4), {}), ("euler", 1, (9,), dict(bc="prescribed", periodic=False)),
+        ("euler", 2, (4, 5), dict(bc="reflect", periodic=(False, True))), ("euler", 3, (3, 2, 3), {}),
+        ("euler_gravity", 2, (3, 4), dict(bc="reflect", periodic=(True, False))),
+        ("euler_gravity", 3, (2, 3, 2), dict(bc="reflect", periodic=False, source="coriolis")),
+        ("euler_gravity", 3, (2, 2, 3), dict(bc="copy", periodic=(True, True, False), level=True)),
+        ("linear_euler_gravity", 2, (3, 4), dict(bc="reflect", periodic=(True, False), directions=(2,),
+                                                 ordering="stacked")),
+        ("linear_euler_gravity", 3, (2, 3, 4), dict(bc="reflect", periodic=(True, True, False), directions=(3,),
+                                                    ordering="stacked")),
+        ("shallow_water", 1, (6,), {}), ("shallow_water", 2, (5, 4), {}), ("shallow_water", 2, (1, 1), {}),
+        ("shallow_water", 3, (2, 3, 2), {}), ("advection", 2, (3, 4), dict(directions=(2,)))]
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("law,dim,Kd,kw", WEAK, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(WEAK)])
+def test_weak_box_kernels_equal_the_general_ones(law, dim, Kd, kw, N):
+    """The same operations in the same order on the same numbers: every value equal (the last node is left
+    out: its MJI differs)."""
+    box, general, q0 = pair(law, dim, N, Kd, seed=N, **kw)
+    assert device_bytes(box) > device_bytes(general)  # the compact geometry was found here, and not there
+    a, b = tendencies(box, general, q0)
+    np.testing.assert_array_equal(a[:, :-1], b[:, :-1])
+
+
+@pytest.mark.parametrize("dim,Kd", [(1, (5,)), (2, (4, 3)), (3, (3, 2, 2))])
+def test_device_built_and_host_built_boxes_agree(dim, Kd):
+    import atum_hip as A
+    hb, _, q0 = pair("euler", dim, 4, Kd, seed=3)
+    db, _, _ = pair("euler", dim, 4, Kd, seed=3, geometry="device")
+    outs = []
+    for dg in (hb, db):
+        q = dg.fieldarray(q0)
+        A.LSRK54(dg, q, 1e-3).run(q, 3)
+        dg.ctx.sync()
+        outs.append(q.numpy())
+    np.testing.assert_array_equal(outs[0], outs[1])
