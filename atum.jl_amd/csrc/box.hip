@@ -212,6 +212,11 @@ Resolved resolve_box_weak_euler_gravity(int dim, int mask, int Nq);
 Resolved resolve_box_weak_linear(int dim, int mask, int Nq);
 Resolved resolve_box_weak_shallow_water(int dim, int mask, int Nq);
 
+Resolved resolve_box_fast_euler_roe(int dim, int Nq);
+Resolved resolve_box_fast_euler_rusanov(int dim, int Nq);
+Resolved resolve_box_fast_euler_gravity_roe(int dim, int Nq);
+Resolved resolve_box_fast_euler_gravity_rusanov(int dim, int Nq);
+
 // Kernels for an operator whose elements are all boxes (fn == nullptr: the general ones)
 Resolved resolve_box(const atm_dg_desc* d, int Nq) {
   if (d->volume_form == ATM_FORM_WEAK && d->surface_flux == ATM_FLUX_RUSANOV) switch (d->law) {
@@ -222,6 +227,16 @@ Resolved resolve_box(const atm_dg_desc* d, int Nq) {
       case ATM_LAW_SHALLOW_WATER: return resolve_box_weak_shallow_water(d->dim, d->dirmask, Nq);
       default: break;
     }
+  if (d->volume_form == ATM_FORM_FLUX_DIFFERENCING && d->volume_flux == ATM_FLUX_EC &&
+      d->precision == ATM_PRECISION_FAST && d->dirmask == (1 << d->dim) - 1) {
+    const bool roe = d->surface_flux == ATM_FLUX_ROE;
+    if (roe || d->surface_flux == ATM_FLUX_RUSANOV) {
+      if (d->law == ATM_LAW_EULER)
+        return roe ? resolve_box_fast_euler_roe(d->dim, Nq) : resolve_box_fast_euler_rusanov(d->dim, Nq);
+      if (d->law == ATM_LAW_EULER_GRAVITY)
+        return roe ? resolve_box_fast_euler_gravity_roe(d->dim, Nq) : resolve_box_fast_euler_gravity_rusanov(d->dim, Nq);
+    }
+  }
   return Resolved{nullptr, 0, 0, nullptr, 1};
 }
 

@@ -1,0 +1,485 @@
+// Pair-symmetric EC flux-differencing kernel (ATM_PRECISION_FAST) on box elements.
+//
+// The operator of fd_fast.hpp with the geometry of a box taken out of the sums.  With a diagonal
+// metric and MJ = J w_i w_j w_k a pair {a, b} of a line in direction r has
+//   MJI_a G_ab = (g_r / w_a) S_ab,   S_ab = D[b,a] w_b - D[a,b] w_a = -S_ba,
+// so a node needs only row r of the two-point flux, one table entry per pair and one factor per
+// direction; MJ, MJI and the metric rows are not read at all.  The surface term scales as
+// faceMJ MJI = g_r / w_end.  A face's flux is evaluated in a frame turned (and for the low face
+// reflected) so that the outward normal is the first axis: the normal's zeros and ones drop out.
+//
+// Work split as in fd_fast.hpp: thread = node, tournament pairing, the partner's share through LDS.
+// The shares of at most SLOTS pair distances are exchanged at a time, which bounds the element's LDS
+// for the high degrees.
+#pragma once
+#include "box.hpp"
+#include "fd_fast.hpp"
+
+namespace atm {
+
+// Pair distances exchanged in one round
+constexpr int BOX_SLOTS = 2;
+
+template <class L, int NQ>
+constexpr int box_xbuf() {
+  constexpr int D = L::D, Ns = L::Ns, Np = ipow(NQ, D), M = NQ / 2;
+  // a round of BOX_SLOTS distances, or all of them; with even NQ the last distance has half the shares
+  constexpr int full = M <= BOX_SLOTS ? (NQ % 2 == 0 ? (M - 1) * Ns * Np + Ns * (Np / 2) : M * Ns * Np)
+                                      : BOX_SLOTS * Ns * Np;
+  constexpr int faces = 2 * D * (Np / NQ) * Ns;
+  return full > faces ? full : faces;
+}
+
+// LDS planes of primitives: [rho, u (D), b, phi (gravity), 1/b (gravity)]
+template <class L>
+constexpr int box_planes() {
+  return L::LAW == ATM_LAW_EULER_GRAVITY ? L::D + 4 : L::D + 2;
+}
+
+template <class L, int NQ>
+constexpr size_t fast_box_elem_doubles() {
+  return (size_t)box_planes<L>() * ipow(NQ, L::D) + box_xbuf<L, NQ>();
+}
+
+// FAST surface flux with the normal along the first momentum component
+template <class L, int SF>
+ATM_DEV void axis_fast_flux(const LawConst& c, const double* qm, double phim, double prefm, const double* qp,
+                            double phip, double prefp, double* nf) {
+  constexpr int D = L::D, Ns = L::Ns;
+  constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
+  // the pressures keep the reference's rounding (fast_flux.hpp)
+  double pm, pfp, pp;
+  if constexpr (GRAV) {
+    pm = L::pressure(c, qm[0], qm + 1, qm[D + 1], phim);
+    pfp = L::pressure(c, qp[0], qp + 1, qp[D + 1], phip);
+    pp = SF == ATM_FLUX_ROE ? L::pressure(c, qp[0], qp + 1, qp[D + 1], phim) : pfp;
+  } else {
+    pm = L::pressure(c, qm[0], qm + 1, qm[D + 1]);
+    pp = pfp = L::pressure(c, qp[0], qp + 1, qp[D + 1]);
+  }
+  {
+#pragma clang fp contract(fast)
+    const double irm = fast_rcp(qm[0]), irp = fast_rcp(qp[0]);
+    double um[D], up[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      um[d] = qm[1 + d] * irm;
+      up[d] = qp[1 + d] * irp;
+    }
+    const double unm = um[0], unp = up[0];
+    // sum of the normal physical fluxes
+    double fs[Ns];
+    fs[0] = qm[1] + qp[1];
+#pragma unroll
+    for (int d = 0; d < D; ++d) fs[1 + d] = qm[1 + d] * unm + qp[1 + d] * unp;
+    fs[1] += (pm - prefm) + (pfp - prefp);
+    fs[D + 1] = unm * (qm[D + 1] + pm) + unp * (qp[D + 1] + pfp);
+    if constexpr (SF == ATM_FLUX_RUSANOV) {
+      const double wm = fabs(unm) + fast_sqrt(c.gamma * pm * irm);
+      const double wp = fabs(unp) + fast_sqrt(c.gamma * pfp * irp);
+      const double ws = 0.5 * fmax(wm, wp);
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) nf[s] = 0.5 * fs[s] - ws * (qp[s] - qm[s]);
+    } else {
+      const double hm = (qm[D + 1] + pm) * irm, hp = (qp[D + 1] + pp) * irp;
+      const double cm = fast_sqrt(c.gamma * pm * irm), cp = fast_sqrt(c.gamma * pp * irp);
+      const double srm = fast_sqrt(qm[0]), srp = fast_sqrt(qp[0]);
+      const double iden = fast_rcp(srm + srp);
+      const double rho = srm * srp;
+      double u[D], du[D], uu = 0, udu = 0;
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        u[d] = (srm * um[d] + srp * up[d]) * iden;
+        du[d] = up[d] - um[d];
+        uu += u[d] * u[d];
+        if (d > 0) udu += u[d] * du[d];  // u.du - (u.n)(du.n)
+      }
+      const double un = u[0], dun = du[0];
+      const double h = (srm * hm + srp * hp) * iden;
+      const double cs = (srm * cm + srp * cp) * iden;
+      const double drho = qp[0] - qm[0], dp = pp - pm;
+      const double cm2 = fast_rcp(cs * cs);
+      const double w1 = 0.5 * fabs(un - cs) * (dp - rho * cs * dun) * cm2;
+      const double w2 = 0.5 * fabs(un + cs) * (dp + rho * cs * dun) * cm2;
+      const double w3 = fabs(un) * (drho - dp * cm2);
+      const double w4 = fabs(un) * rho;
+      const double e3 = GRAV ? w3 * (0.5 * uu + phim) : 0.5 * w3 * uu;
+      const double ws = w1 + w2 + w3, wc = cs * (w2 - w1);
+      nf[0] = 0.5 * fs[0] - 0.5 * ws;
+      nf[1] = 0.5 * fs[1] - 0.5 * (ws * u[0] + wc);
+#pragma unroll
+      for (int d = 1; d < D; ++d) nf[1 + d] = 0.5 * fs[1 + d] - 0.5 * (ws * u[d] + w4 * du[d]);
+      nf[D + 1] = 0.5 * fs[D + 1] - 0.5 * ((w1 + w2) * h + wc * un + e3 + w4 * udu);
+    }
+  }
+}
+
+// The face points of an element dealt out over its threads (FastFaces of fd_fast.hpp): point
+// f = t + i Np in round i; buf[s * NFP + f] takes the flux times g_r / w_end.
+template <class L, int SF, int NQ>
+struct BoxFaces {
+  static constexpr int D = L::D, Ns = L::Ns, Np = ipow(NQ, D), NFPF = Np / NQ, NFP = 2 * D * NFPF;
+  static constexpr int R = (NFP + Np - 1) / Np;  // rounds
+  static constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
+  int nb[R];  // neighbour element or minus the boundary tag
+  // a round past the last face point reads the last face's entry and ignores it
+  ATM_DEV void load(const BoxElem<D>* rec, int t) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) nb[i] = rec->nb[min(t + i * Np, NFP - 1) / NFPF];
+  }
+  // sQ: [s][node] the element's state and, for Euler-gravity, its geopotential (s = Ns); lift: g_r / w_end
+  ATM_DEV void run(const DevDG& p, int64_t e, int t, const double* q, double* buf, const double* sQ,
+                   const double* lift) const {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int f = t + i * Np;
+      if (f >= NFP) break;
+      const int face = f / NFPF, fp = f - face * NFPF, r = face >> 1;
+      const bool hi = face & 1;
+      const int st = r == 0 ? 1 : (r == 1 ? NQ : NQ * NQ);
+      // face point -> node: the coordinates below direction r, then those above it
+      const int low = fp % st, ln0 = low + (fp - low) * NQ;
+      const int ln = ln0 + (hi ? (NQ - 1) * st : 0);
+      // a boundary face point reads its own node as the neighbour (every load unconditional)
+      const int64_t idp = nb[i] >= 0 ? (int64_t)nb[i] * Np + ln0 + (hi ? 0 : (NQ - 1) * st) : e * Np + ln;
+      const double sg = hi ? 1.0 : -1.0;
+      int pl[D];  // state planes of the turned momentum components
+#pragma unroll
+      for (int d = 0; d < D; ++d) pl[d] = 1 + (r + d >= D ? r + d - D : r + d);
+      double qp[Ns], qm[Ns], nf[Ns];
+      qp[0] = q[idp];
+#pragma unroll
+      for (int d = 0; d < D; ++d) qp[1 + d] = q[pl[d] * p.Ntot + idp];
+      qp[D + 1] = q[(D + 1) * p.Ntot + idp];
+      const double phip0 = GRAV ? p.aux[idp] : 0.0;
+      qm[0] = sQ[ln];
+#pragma unroll
+      for (int d = 0; d < D; ++d) qm[1 + d] = sQ[pl[d] * Np + ln];
+      qm[D + 1] = sQ[(D + 1) * Np + ln];
+      const double phim = GRAV ? sQ[Ns * Np + ln] : 0.0;
+      double phip = phip0;
+      double prefm = 0.0, prefp = 0.0;
+      if (GRAV && p.c.pde_level_balance) {  // uniform over the launch
+        prefm = p.aux[(D + 2) * p.Ntot + e * Np + ln];
+        prefp = p.aux[(D + 2) * p.Ntot + idp];
+      }
+      qm[1] *= sg;
+      qp[1] *= sg;
+      if (nb[i] < 0) {
+        phip = phim;
+        prefp = prefm;
+        if (p.c.bc == ATM_BC_REFLECT) {
+#pragma unroll
+          for (int s = 0; s < Ns; ++s) qp[s] = qm[s];
+          qp[1] = qm[1] - 2 * qm[1];
+        } else {
+          // the other boundary states are defined in the mesh frame
+          double n[D], qo[Ns], qb[Ns];
+#pragma unroll
+          for (int d = 0; d < D; ++d) n[d] = d == r ? sg : 0.0;
+#pragma unroll
+          for (int s = 0; s < Ns; ++s) qo[s] = sQ[s * Np + ln];
+          boundarystate<L>(p.c, n, qo, -nb[i], qb);
+          qp[0] = qb[0];
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            double v = qb[1];
+#pragma unroll
+            for (int k = 1; k < D; ++k) v = pl[d] == 1 + k ? qb[1 + k] : v;
+            qp[1 + d] = v;
+          }
+          qp[1] *= sg;
+          qp[D + 1] = qb[D + 1];
+        }
+      }
+      axis_fast_flux<L, SF>(p.c, qm, phim, prefm, qp, phip, prefp, nf);
+      nf[1] *= sg;
+      double lf = lift[0];
+#pragma unroll
+      for (int d = 1; d < D; ++d) lf = r == d ? lift[d] : lf;
+      buf[f] = lf * nf[0];
+#pragma unroll
+      for (int d = 0; d < D; ++d) buf[pl[d] * NFP + f] = lf * nf[1 + d];
+      buf[(D + 1) * NFP + f] = lf * nf[D + 1];
+    }
+  }
+  ATM_DEV static void gather(const int idx[3], const double* buf, double* acc) {
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+      const int ir = idx[r];
+      if (ir != 0 && ir != NQ - 1) continue;
+      int fp = 0;
+      if (D == 2) fp = (r == 0) ? idx[1] : idx[0];
+      if (D == 3) fp = (r == 0) ? idx[1] + NQ * idx[2] : ((r == 1) ? idx[0] + NQ * idx[2] : idx[0] + NQ * idx[1]);
+      const int f = (2 * r + (ir != 0)) * NFPF + fp;
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) acc[s] -= buf[s * NFP + f];
+    }
+  }
+};
+
+template <class L, int NQ, int SF>
+ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
+                           double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
+                           int epw) {
+#pragma clang fp contract(fast)
+  constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
+  using FE = FastEC<L::D, GRAV>;
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D), M = NQ / 2, NPL = box_planes<L>();
+  constexpr bool HALF = NQ % 2 == 0;  // the pairs at distance NQ/2 are taken by the lower half of each line
+  constexpr int stride = (int)fast_box_elem_doubles<L, NQ>();
+  static_assert(NPL >= Ns + (GRAV ? 1 : 0), "the surface term stages the state in the primitives' planes");
+  double* sS = lds;                // S_ab at [b + NQ a]
+  double* siw = lds + NQ * NQ;     // 1 / w_a
+  const int tid = threadIdx.x;
+  const int el = tid / Np;
+  const int ijk = tid - el * Np;
+  const int64_t le = blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < p.K;
+  const int64_t e = (p.sched && active) ? (int64_t)p.sched[le] : le;
+  double* sP = lds + NQ * NQ + NQ + el * stride;  // [k][node]
+  double* sx = sP + NPL * Np;                     // [slot][s][node]
+  for (int t = tid; t < NQ * NQ; t += blockDim.x) {
+    const int b = t % NQ, a = t / NQ;
+    sS[t] = p.D[b + NQ * a] * p.bw[b] - p.D[a + NQ * b] * p.bw[a];
+  }
+  for (int t = tid; t < NQ; t += blockDim.x) siw[t] = 1 / p.bw[t];
+  // every load of the node's data first and unconditionally (a lane past the last element reads
+  // element 0 and discards it)
+  const int64_t e0 = active ? e : 0;
+  const int64_t node = e0 * Np + ijk;
+  const BoxElem<D>* rec = &box_elem<D>(p, e0);
+  double q1[Ns], a1[NA], P1[FE::NP];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) q1[s] = q[s * p.Ntot + node];
+  load_aux<L>(p, node, a1);
+  double g[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) g[d] = rec->g[d];
+  using BF = BoxFaces<L, SF, NQ>;
+  BF bf;
+  bf.load(rec, ijk);
+  FE::prim(p.c, q1, a1, P1);
+  if (active) {
+#pragma unroll
+    for (int k = 0; k < D + 2; ++k) sP[k * Np + ijk] = P1[k];
+    if constexpr (GRAV) {
+      sP[(D + 2) * Np + ijk] = P1[D + 3];
+      sP[(D + 3) * Np + ijk] = P1[D + 4];
+    }
+  }
+  int idx[3];
+  node_index<D>(ijk, NQ, idx);
+  // a node of the upper half of its line in direction r, at line position c >= M, by its position there
+  auto half_pos = [&](int r, int c) {
+    int pos = 0, st = 1;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      pos += (d == r ? c - M : idx[d]) * st;
+      st *= d == r ? M : NQ;
+    }
+    return pos;
+  };
+  const double inv_gm1 = 1 / (p.c.gamma - 1);
+  double acc[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) acc[s] = 0.0;
+  if (active) L::sources(p.c, acc, q1, a1, all_dirs<L>(), false);
+  __syncthreads();  // tables and primitives written
+#pragma unroll
+  for (int r = 0; r < D; ++r) {
+    const int a = idx[r];
+    const int st = r == 0 ? 1 : (r == 1 ? NQ : NQ * NQ);
+    const int lbase = ijk - a * st;
+    double vol[Ns];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) vol[s] = 0.0;
+#pragma unroll
+    for (int m0 = 1; m0 <= M; m0 += BOX_SLOTS) {
+      if (r > 0 || m0 > 1) __syncthreads();  // the previous round's shares are gathered
+      if (active) {
+#pragma unroll
+        for (int m = m0; m < m0 + BOX_SLOTS && m <= M; ++m) {
+          if (HALF && m == M && a >= M) continue;
+          const int b = a + m >= NQ ? a + m - NQ : a + m;
+          const int ib = lbase + b * st;
+          double P2[FE::NP];
+#pragma unroll
+          for (int k = 0; k < D + 2; ++k) P2[k] = sP[k * Np + ib];
+          P2[D + 2] = P2[1] * P2[1];
+#pragma unroll
+          for (int d = 1; d < D; ++d) P2[D + 2] += P2[1 + d] * P2[1 + d];
+          P2[D + 3] = GRAV ? sP[(D + 2) * Np + ib] : 0.0;
+          P2[D + 4] = GRAV ? sP[(D + 3) * Np + ib] : 0.0;
+          typename FE::Pair w;
+          FE::pair(p.c, inv_gm1, P1, P2, w);
+          const double S = sS[b + NQ * a];
+          // S times row r of the symmetric part of the flux
+          double sf[Ns];
+          const double su = S * w.u[r];
+          sf[0] = w.rho_log * su;
+#pragma unroll
+          for (int d = 0; d < D; ++d) sf[1 + d] = w.u[d] * sf[0];
+          sf[1 + r] += w.pd * S;
+          sf[D + 1] = su * w.ecoef;
+#pragma unroll
+          for (int s = 0; s < Ns; ++s) vol[s] += sf[s];
+          if (GRAV) vol[1 + r] -= S * w.fla;
+          // the partner's share, which it subtracts
+          const bool hs = HALF && m == M;
+          double* slot = sx + (m - m0) * Ns * Np + (hs ? half_pos(r, b) : ib);
+          const int xs = hs ? Np / 2 : Np;
+          if (GRAV) sf[1 + r] -= S * w.flb;
+#pragma unroll
+          for (int s = 0; s < Ns; ++s) slot[s * xs] = sf[s];
+        }
+      }
+      __syncthreads();
+      if (active) {
+#pragma unroll
+        for (int m = m0; m < m0 + BOX_SLOTS && m <= M; ++m) {
+          if (HALF && m == M && a < M) continue;
+          const bool hs = HALF && m == M;
+          const double* slot = sx + (m - m0) * Ns * Np + (hs ? half_pos(r, a) : ijk);
+          const int xs = hs ? Np / 2 : Np;
+#pragma unroll
+          for (int s = 0; s < Ns; ++s) vol[s] -= slot[s * xs];
+        }
+      }
+    }
+    const double gw = g[r] * siw[a];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) acc[s] += gw * vol[s];
+  }
+  // Surface term: no thread reads a partner's primitives any more, so the state and geopotential are
+  // staged by node in their planes; the face points read their own side there, the update the state.
+  double* sQ = sP;
+  if (active) {
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) sQ[s * Np + ijk] = q[s * p.Ntot + node];
+    if constexpr (GRAV) sQ[Ns * Np + ijk] = P1[D + 3];
+  }
+  double lift[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) lift[d] = g[d] * siw[0];
+  __syncthreads();  // every thread has consumed its exchange slots
+  if (active) bf.run(p, e, ijk, q, sx, sQ, lift);
+  __syncthreads();
+  if (!active) return;
+  double dq0[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) dq0[s] = assign ? 0.0 : dq[s * p.Ntot + node];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) q1[s] = sQ[s * Np + ijk];
+  if (!assign) {
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) acc[s] += alpha * dq0[s];
+  }
+  BF::gather(idx, sx, acc);
+  epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+}
+
+template <class L, int NQ, int SF>
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, fast_max_threads<L, NQ, SF>())))
+fast_box_kernel(const DevDG p, const double* __restrict__ q, double* __restrict__ dq, double alpha, int assign,
+                double* __restrict__ qout, double bdt, int epw) {
+  extern __shared__ double lds[];
+  fast_box_body<L, NQ, SF>(p, lds, xcd_block(), q, dq, alpha, assign, qout, bdt, epw);
+}
+
+template <class L, int NQ, int SF>
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, fast_max_threads<L, NQ, SF>())))
+fast_box_kernel_batch(const BatchEntry* __restrict__ tab, int n, int parity, double alpha, int assign, double b,
+                      int epw) {
+  extern __shared__ double lds[];
+  const int64_t lb = xcd_block();
+  const int i = batch_find(tab, n, lb);
+  const DevDG p = tab[i].p;
+  fast_box_body<L, NQ, SF>(p, lds, lb - tab[i].block_start, tab[i].buf[parity], tab[i].dq, alpha, assign,
+                           tab[i].buf[1 - parity], b * tab[i].dt, epw);
+}
+
+// One launch per stage for members of N = 3..7 (as fd_fast_multi_kernel_batch)
+template <class L, int SF>
+__global__ void __launch_bounds__(512)
+    fast_box_multi_kernel_batch(const BatchEntry* __restrict__ tab, int n, int parity, double alpha, int assign,
+                                double b) {
+  extern __shared__ double lds[];
+  const int64_t lb = xcd_block();
+  const int i = batch_find(tab, n, lb);
+  const DevDG p = tab[i].p;
+  const int64_t blk = lb - tab[i].block_start;
+  const double* qin = tab[i].buf[parity];
+  double* qo = tab[i].buf[1 - parity];
+  const double bdt = b * tab[i].dt;
+  switch (p.Nq) {
+    case 4: fast_box_body<L, 4, SF>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 5: fast_box_body<L, 5, SF>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 6: fast_box_body<L, 6, SF>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 7: fast_box_body<L, 7, SF>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    case 8: fast_box_body<L, 8, SF>(p, lds, blk, qin, tab[i].dq, alpha, assign, qo, bdt, p.epw); break;
+    default: break;
+  }
+}
+
+template <class L, int SF>
+hipError_t launch_fast_box_multi_batch(const BatchEntry* tab, int n, int64_t blocks, int threads, size_t lds, int epw,
+                                       hipStream_t st, int parity, double alpha, int assign, double b) {
+  (void)epw;  // every member carries its own in the table
+  hipLaunchKernelGGL((fast_box_multi_kernel_batch<L, SF>), dim3(blocks), dim3(threads), lds, st, tab, n, parity, alpha,
+                     assign, b);
+  return hipGetLastError();
+}
+
+template <class L, int NQ, int SF>
+hipError_t launch_fast_box(const DevDG& p, hipStream_t st, const double* q, double* dq, double alpha, int assign,
+                           double* qout, double bdt) {
+  constexpr int Np = ipow(NQ, L::D);
+  const int threads = ((p.epw * Np + 63) / 64) * 64;
+  if (p.epw < 1 || threads > fast_max_threads<L, NQ, SF>()) return hipErrorInvalidConfiguration;
+  const int blocks = (p.K + p.epw - 1) / p.epw;
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL((fast_box_kernel<L, NQ, SF>), dim3(blocks), dim3(threads), p.lds, st, p, q, dq, alpha, assign,
+                     qout, bdt, p.epw);
+  return hipGetLastError();
+}
+
+template <class L, int NQ, int SF>
+hipError_t launch_fast_box_batch(const BatchEntry* tab, int n, int64_t blocks, int threads, size_t lds, int epw,
+                                 hipStream_t st, int parity, double alpha, int assign, double b) {
+  hipLaunchKernelGGL((fast_box_kernel_batch<L, NQ, SF>), dim3(blocks), dim3(threads), lds, st, tab, n, parity, alpha,
+                     assign, b, epw);
+  return hipGetLastError();
+}
+
+template <class L, int NQ, int SF>
+Resolved fast_box_variant() {
+  Resolved r = make_resolved(launch_fast_box<L, NQ, SF>, launch_fast_box_batch<L, NQ, SF>, L::Ns,
+                             fast_epw<L, NQ, SF>(), sizeof(double) * (NQ * NQ + NQ),
+                             sizeof(double) * fast_box_elem_doubles<L, NQ>(), fast_max_threads<L, NQ, SF>());
+  if constexpr (NQ >= 4 && NQ <= 8) r.mbfn = launch_fast_box_multi_batch<L, SF>;
+  return r;
+}
+
+template <class L, int SF>
+Resolved fast_box_nq(int Nq) {
+  switch (Nq) {
+    case 2: return fast_box_variant<L, 2, SF>();
+    case 3: return fast_box_variant<L, 3, SF>();
+    case 4: return fast_box_variant<L, 4, SF>();
+    case 5: return fast_box_variant<L, 5, SF>();
+    case 6: return fast_box_variant<L, 6, SF>();
+    case 7: return fast_box_variant<L, 7, SF>();
+    case 8: return fast_box_variant<L, 8, SF>();
+    default: return Resolved{nullptr, 0, 0, nullptr, 1};
+  }
+}
+
+template <template <int> class LAW, int SF>
+Resolved fast_box_dims(int dim, int Nq) {
+  if (dim == 2) return fast_box_nq<LAW<2>, SF>(Nq);
+  if (dim == 3) return fast_box_nq<LAW<3>, SF>(Nq);
+  return Resolved{nullptr, 0, 0, nullptr, 1};
+}
+
+}  // namespace atm

@@ -1,0 +1,6 @@
+// Pair-symmetric EC flux-differencing kernels on box elements for EulerGravityLaw, roe surface flux.
+#include "box_fast.hpp"
+
+namespace atm {
+Resolved resolve_box_fast_euler_gravity_roe(int dim, int Nq) { return fast_box_dims<EulerGravity, ATM_FLUX_ROE>(dim, Nq); }
+}  // namespace atm

@@ -18,8 +18,9 @@ def pair(law, dim, N, Kd, form="weak", sflux="rusanov", bc="copy", periodic=True
     size = 2000.0 if "gravity" in law else 2.0
     coords = [np.concatenate([[0.0], np.cumsum(rng.uniform(0.7, 1.3, k))]) * size / k for k in Kd]
     per = (periodic,) * dim if isinstance(periodic, bool) else periodic
-    prob = A.Problem(boundary=bc, source=source, omega=1e-2,
-                     bc_states=rng.uniform(1, 2, (2 * dim, dim + 2)) if bc == "prescribed" else None)
+    states = rng.uniform(1, 2, (2 * dim, dim + 2))
+    states[:, -1] += 8  # positive pressure
+    prob = A.Problem(boundary=bc, source=source, omega=1e-2, bc_states=states if bc == "prescribed" else None)
     u = (1.0, -0.4, 0.7)[:dim]
 
     def build(off):
@@ -102,3 +103,22 @@ def test_device_built_and_host_built_boxes_agree(dim, Kd):
         dg.ctx.sync()
         outs.append(q.numpy())
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+FAST = [("euler", 2, (4, 3), dict(bc="prescribed", periodic=False)), ("euler", 2, (3, 5), {}),
+        ("euler", 3, (2, 3, 2), dict(bc="reflect", periodic=(False, True, False))),
+        ("euler_gravity", 2, (3, 4), dict(bc="reflect", periodic=(True, False), level=True)),
+        ("euler_gravity", 3, (2, 2, 3), dict(bc="reflect", periodic=False, source="coriolis")),
+        ("euler_gravity", 3, (3, 2, 2), dict(bc="copy", periodic=(True, False, False), ordering="stacked"))]
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("sflux", ["roe", "rusanov"])
+@pytest.mark.parametrize("law,dim,Kd,kw", FAST, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(FAST)])
+def test_fast_box_kernels_against_the_general_ones(law, dim, Kd, kw, sflux, N):
+    """Another order of the same sums: each form is within 1e-12 of the oracle's tendency (relative
+    max-norm, tests/test_gpu_fast.py), so they are within 2e-12 of each other."""
+    box, general, q0 = pair(law, dim, N, Kd, form="ec", sflux=sflux, precision="fast", seed=10 + N, **kw)
+    assert device_bytes(box) > device_bytes(general)
+    a, b = tendencies(box, general, q0)
+    assert np.abs(a - b).max() <= 2e-12 * np.abs(b).max()
