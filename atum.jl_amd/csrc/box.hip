@@ -147,7 +147,7 @@ namespace atm {
 
 int dg_box(atm_dg* dg, const atm_dg_desc* d, const double* w_host) {
   DevDG& p = dg->dev;
-  if (p.K < 1) return ATM_OK;
+  if (p.K < 1 || dg->Ns * dg->Ntot >= BOX_MAX_STATE) return ATM_OK;
   const Resolved r = resolve_box(d, dg->Nq);
   atm_ctx* ctx = dg->ctx;
   if (!r.fn || r.lds > ctx->max_lds) return ATM_OK;

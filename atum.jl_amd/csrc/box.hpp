@@ -26,9 +26,50 @@ struct BoxElem {
   int32_t nb[2 * D];  // neighbour element of each face, or minus the boundary tag
 };
 
+// The box kernels address fields with 32-bit byte offsets from a uniform base (a scalar register and
+// one vector register per address instead of 64-bit vector arithmetic for every load), so they take
+// operators whose state is below 4 GB; larger ones run the general kernels.
+constexpr int64_t BOX_MAX_STATE = (int64_t)1 << 29;  // doubles
+
+// A global pointer kept in scalar registers: the empty statement hides it from the address arithmetic
+// of the lanes, so that a load takes it as the base and the lane's offset as one register.
+typedef const char __attribute__((address_space(1))) * gptr;
+ATM_DEV gptr uniform(const void* b) {
+  gptr g = (gptr)b;
+  asm("" : "+s"(g));
+  return g;
+}
+ATM_DEV double ldg(gptr b, uint32_t off) { return *(const double __attribute__((address_space(1)))*)(b + off); }
+ATM_DEV void stg(gptr b, uint32_t off, double v) { *(double __attribute__((address_space(1)))*)(char __attribute__((address_space(1)))*)(b + off) = v; }
+
+// component s of a field at a byte offset
+ATM_DEV double ldo(const DevDG& p, const double* field, int s, uint32_t off) {
+  return ldg(uniform(field + s * p.Ntot), off);
+}
+ATM_DEV void sto(const DevDG& p, double* field, int s, uint32_t off, double v) {
+  stg(uniform(field + s * p.Ntot), off, v);
+}
+
 template <int D>
-ATM_DEV const BoxElem<D>& box_elem(const DevDG& p, int64_t e) {
-  return static_cast<const BoxElem<D>*>(p.box)[e];
+ATM_DEV const BoxElem<D>* box_elem(const DevDG& p, uint32_t e) {
+  return reinterpret_cast<const BoxElem<D>*>(static_cast<const char*>(p.box) + e * (uint32_t)sizeof(BoxElem<D>));
+}
+
+// load_aux and epilogue with a byte offset of the node
+template <class L>
+ATM_DEV void box_aux(const DevDG& p, uint32_t off, double* a) {
+#pragma unroll
+  for (int s = 0; s < L::NA; ++s) a[s] = (s < p.naux) ? ldo(p, p.aux, s, off) : 0.0;
+}
+
+template <class L>
+ATM_DEV void box_epilogue(const DevDG& p, uint32_t off, const double* q1, const double* acc, double* __restrict__ dq,
+                          double* __restrict__ qout, double bdt) {
+#pragma unroll
+  for (int s = 0; s < L::Ns; ++s) {
+    sto(p, dq, s, off, acc[s]);
+    if (qout) sto(p, qout, s, off, q1[s] + bdt * acc[s]);
+  }
 }
 
 constexpr int ipow(int b, int n) { return n == 0 ? 1 : b * ipow(b, n - 1); }
@@ -101,7 +142,7 @@ ATM_DEV void axis_surfaceflux(const LawConst& c, double sg, const double* qm, co
 // Surface contributions of the faces this node lies on, subtracted from acc (surface_node on
 // box elements).  sw: the LGL weights.
 template <class L, int SF, int NQ, int MASK>
-ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, int64_t e, int ijk, const int idx[3],
+ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, uint32_t e, int ijk, const int idx[3],
                               const double* q, const double* qn, const double* an, double MJIn, const double* sw,
                               double* acc) {
   constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D);
@@ -114,11 +155,11 @@ ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, int64_t e,
     const int nb = hi ? b.nb[2 * r + 1] : b.nb[2 * r];
     constexpr int span = (NQ - 1) * line_stride<NQ, r>();
     // a boundary node reads its own state as the neighbour's and replaces it by the boundary state
-    const int64_t idp = nb >= 0 ? (int64_t)nb * Np + ijk + (hi ? -span : span) : e * Np + ijk;
+    const uint32_t idp = 8 * (nb >= 0 ? (uint32_t)nb * Np + ijk + (hi ? -span : span) : e * Np + ijk);
     double qp[Ns], ap[NA], nf[Ns];
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) qp[s] = q[s * p.Ntot + idp];
-    load_aux<L>(p, idp, ap);
+    for (int s = 0; s < Ns; ++s) qp[s] = ldo(p, q, s, idp);
+    box_aux<L>(p, idp, ap);
     const double sg = hi ? 1.0 : -1.0;
     if (nb < 0) {
       double n[D];
@@ -157,29 +198,29 @@ ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   const int tid = threadIdx.x;
   const int el = tid / Np;
   const int ijk = tid - el * Np;
-  const int64_t le = blk * epw + el;  // position in the processing order
-  const bool active = el < epw && le < p.K;
-  const int64_t e = (p.sched && active) ? (int64_t)p.sched[le] : le;
+  const uint32_t le = (uint32_t)blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < (uint32_t)p.K;
+  const uint32_t e = (p.sched && active) ? (uint32_t)p.sched[le] : le;
   double* slF = lds + NQ * NQ + NQ + el * (dirs * Ns * Np);  // [dir slot][s][node]
   for (int t = tid; t < NQ * NQ; t += blockDim.x) sD[t] = p.D[t];
   for (int t = tid; t < NQ; t += blockDim.x) sw[t] = p.bw[t];
   double q1[Ns], a1[NA];
-  const int64_t el_e = active ? e : 0;  // a lane past the last element reads element 0 and discards it
-  const int64_t node = el_e * Np + ijk;
+  const uint32_t el_e = active ? e : 0;  // a lane past the last element reads element 0 and discards it
+  const uint32_t node = 8 * (el_e * Np + ijk);
   int idx[3];
   node_index<D>(ijk, NQ, idx);
   // every load first and unconditionally: the element's record, state, aux and the stage's dq in flight together
-  const BoxElem<D> b = box_elem<D>(p, el_e);
+  const BoxElem<D> b = *box_elem<D>(p, el_e);
 #pragma unroll
-  for (int s = 0; s < Ns; ++s) q1[s] = q[s * p.Ntot + node];
-  load_aux<L>(p, node, a1);
+  for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
+  box_aux<L>(p, node, a1);
   const double wp = p.bw[NQ + ijk];
   double dq0[Ns];
 #pragma unroll
   for (int s = 0; s < Ns; ++s) dq0[s] = 0.0;
   if (!assign) {  // uniform over the launch
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) dq0[s] = dq[s * p.Ntot + node];
+    for (int s = 0; s < Ns; ++s) dq0[s] = ldo(p, dq, s, node);
   }
   const double MJn = wp * b.J;
   if (active) {
@@ -224,7 +265,7 @@ ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
 #pragma unroll
   for (int s = 0; s < Ns; ++s) acc[s] = assign ? dl[s] : alpha * dq0[s] + dl[s];
   box_surface_node<L, SF, NQ, MASK>(p, b, e, ijk, idx, q, q1, a1, MJIn, sw, acc);
-  epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+  box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
 }
 
 ATM_KERNEL_PAIR(weak_box_kernel, weak_box_body, class L ATM_COMMA int NQ ATM_COMMA int SF ATM_COMMA int MASK,

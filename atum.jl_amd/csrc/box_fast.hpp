@@ -127,9 +127,9 @@ struct BoxFaces {
 #pragma unroll
     for (int i = 0; i < R; ++i) nb[i] = rec->nb[min(t + i * Np, NFP - 1) / NFPF];
   }
-  // sQ: [s][node] the element's state and, for Euler-gravity, its geopotential (s = Ns); lift: g_r / w_end
-  ATM_DEV void run(const DevDG& p, int64_t e, int t, const double* q, double* buf, const double* sQ,
-                   const double* lift) const {
+  // sQ: [s][node] the element's state and, for Euler-gravity, its geopotential (s = Ns); iw: 1 / w_end
+  ATM_DEV void run(const DevDG& p, const BoxElem<D>* rec, uint32_t e, int t, const double* q, double* buf,
+                   const double* sQ, double iw) const {
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int f = t + i * Np;
@@ -141,17 +141,20 @@ struct BoxFaces {
       const int low = fp % st, ln0 = low + (fp - low) * NQ;
       const int ln = ln0 + (hi ? (NQ - 1) * st : 0);
       // a boundary face point reads its own node as the neighbour (every load unconditional)
-      const int64_t idp = nb[i] >= 0 ? (int64_t)nb[i] * Np + ln0 + (hi ? 0 : (NQ - 1) * st) : e * Np + ln;
+      const uint32_t own = 8 * (e * Np + ln);
+      const uint32_t idp = nb[i] >= 0 ? 8 * ((uint32_t)nb[i] * Np + ln0 + (hi ? 0 : (NQ - 1) * st)) : own;
+      const uint32_t plane = 8 * (uint32_t)p.Ntot;
       const double sg = hi ? 1.0 : -1.0;
+      const double lf = rec->g[r] * iw;
       int pl[D];  // state planes of the turned momentum components
 #pragma unroll
       for (int d = 0; d < D; ++d) pl[d] = 1 + (r + d >= D ? r + d - D : r + d);
       double qp[Ns], qm[Ns], nf[Ns];
-      qp[0] = q[idp];
+      qp[0] = ldo(p, q, 0, idp);
 #pragma unroll
-      for (int d = 0; d < D; ++d) qp[1 + d] = q[pl[d] * p.Ntot + idp];
-      qp[D + 1] = q[(D + 1) * p.Ntot + idp];
-      const double phip0 = GRAV ? p.aux[idp] : 0.0;
+      for (int d = 0; d < D; ++d) qp[1 + d] = ldo(p, q, 0, idp + pl[d] * plane);
+      qp[D + 1] = ldo(p, q, D + 1, idp);
+      const double phip0 = GRAV ? ldo(p, p.aux, 0, idp) : 0.0;
       qm[0] = sQ[ln];
 #pragma unroll
       for (int d = 0; d < D; ++d) qm[1 + d] = sQ[pl[d] * Np + ln];
@@ -160,8 +163,8 @@ struct BoxFaces {
       double phip = phip0;
       double prefm = 0.0, prefp = 0.0;
       if (GRAV && p.c.pde_level_balance) {  // uniform over the launch
-        prefm = p.aux[(D + 2) * p.Ntot + e * Np + ln];
-        prefp = p.aux[(D + 2) * p.Ntot + idp];
+        prefm = ldo(p, p.aux, D + 2, own);
+        prefp = ldo(p, p.aux, D + 2, idp);
       }
       qm[1] *= sg;
       qp[1] *= sg;
@@ -194,9 +197,6 @@ struct BoxFaces {
       }
       axis_fast_flux<L, SF>(p.c, qm, phim, prefm, qp, phip, prefp, nf);
       nf[1] *= sg;
-      double lf = lift[0];
-#pragma unroll
-      for (int d = 1; d < D; ++d) lf = r == d ? lift[d] : lf;
       buf[f] = lf * nf[0];
 #pragma unroll
       for (int d = 0; d < D; ++d) buf[pl[d] * NFP + f] = lf * nf[1 + d];
@@ -234,9 +234,9 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   const int tid = threadIdx.x;
   const int el = tid / Np;
   const int ijk = tid - el * Np;
-  const int64_t le = blk * epw + el;  // position in the processing order
-  const bool active = el < epw && le < p.K;
-  const int64_t e = (p.sched && active) ? (int64_t)p.sched[le] : le;
+  const uint32_t le = (uint32_t)blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < (uint32_t)p.K;
+  const uint32_t e = (p.sched && active) ? (uint32_t)p.sched[le] : le;
   double* sP = lds + NQ * NQ + NQ + el * stride;  // [k][node]
   double* sx = sP + NPL * Np;                     // [slot][s][node]
   for (int t = tid; t < NQ * NQ; t += blockDim.x) {
@@ -246,13 +246,13 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   for (int t = tid; t < NQ; t += blockDim.x) siw[t] = 1 / p.bw[t];
   // every load of the node's data first and unconditionally (a lane past the last element reads
   // element 0 and discards it)
-  const int64_t e0 = active ? e : 0;
-  const int64_t node = e0 * Np + ijk;
-  const BoxElem<D>* rec = &box_elem<D>(p, e0);
+  const uint32_t e0 = active ? e : 0;
+  const uint32_t node = 8 * (e0 * Np + ijk);
+  const BoxElem<D>* rec = box_elem<D>(p, e0);
   double q1[Ns], a1[NA], P1[FE::NP];
 #pragma unroll
-  for (int s = 0; s < Ns; ++s) q1[s] = q[s * p.Ntot + node];
-  load_aux<L>(p, node, a1);
+  for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
+  box_aux<L>(p, node, a1);
   double g[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) g[d] = rec->g[d];
@@ -349,26 +349,26 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
     }
     const double gw = g[r] * siw[a];
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) acc[s] += gw * vol[s];
+    for (int s = 0; s < Ns; ++s) {
+      acc[s] += gw * vol[s];
+      asm("" : "+v"(acc[s]));  // summed here: the compiler would keep every direction's vol until the end
+    }
   }
   // Surface term: no thread reads a partner's primitives any more, so the state and geopotential are
   // staged by node in their planes; the face points read their own side there, the update the state.
   double* sQ = sP;
   if (active) {
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) sQ[s * Np + ijk] = q[s * p.Ntot + node];
+    for (int s = 0; s < Ns; ++s) sQ[s * Np + ijk] = ldo(p, q, s, node);
     if constexpr (GRAV) sQ[Ns * Np + ijk] = P1[D + 3];
   }
-  double lift[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) lift[d] = g[d] * siw[0];
   __syncthreads();  // every thread has consumed its exchange slots
-  if (active) bf.run(p, e, ijk, q, sx, sQ, lift);
+  if (active) bf.run(p, rec, e, ijk, q, sx, sQ, siw[0]);
   __syncthreads();
   if (!active) return;
   double dq0[Ns];
 #pragma unroll
-  for (int s = 0; s < Ns; ++s) dq0[s] = assign ? 0.0 : dq[s * p.Ntot + node];
+  for (int s = 0; s < Ns; ++s) dq0[s] = assign ? 0.0 : ldo(p, dq, s, node);
 #pragma unroll
   for (int s = 0; s < Ns; ++s) q1[s] = sQ[s * Np + ijk];
   if (!assign) {
@@ -376,7 +376,7 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
     for (int s = 0; s < Ns; ++s) acc[s] += alpha * dq0[s];
   }
   BF::gather(idx, sx, acc);
-  epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+  box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
 }
 
 template <class L, int NQ, int SF>
