@@ -30,15 +30,105 @@ constexpr int box_xbuf() {
   return full > faces ? full : faces;
 }
 
-// LDS planes of primitives: [rho, u (D), b, phi (gravity), 1/b (gravity)]
+// Entropy-conservative two-point flux of the Euler laws from per-node primitives
+// [rho, u/2 (D), b = rho/2p, phi/2 (gravity), 1/2b (gravity)]: row r of twice the flux.  With
+// rl = 2 rho_log, pd = 2 rho_avg / 2 b_avg and u the pair average,
+//   F_r = [rl u_r, rl u_r u + pd e_r, u_r (rl (1/(2 (gamma-1) b_log) + phi_avg + u_a.u_b/2) + pd)]
+// (|u|^2 - |u|^2_avg/2 of the reference's energy flux is u_a.u_b/2), and the gravity fluctuation of node
+// a takes t / 2b_a, t = 2 b_avg rl (phi_a - phi_b)/2, from its momentum.  Halved velocities and potentials
+// and the factor 2, which the table S_ab takes back, save the multiplications by 1/2 in every mean.
 template <class L>
-constexpr int box_planes() {
-  return L::LAW == ATM_LAW_EULER_GRAVITY ? L::D + 4 : L::D + 2;
-}
+struct BoxEC {
+  static constexpr int D = L::D, Ns = L::Ns;
+  static constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
+  static constexpr int NP = GRAV ? D + 4 : D + 2;  // LDS planes
+  ATM_DEV static void prim(const LawConst& c, const double* q, double phi, double* P) {
+#pragma clang fp contract(fast)
+    const double ir = fast_rcp(q[0]), hr = 0.5 * ir;
+    double ke = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      P[1 + d] = q[1 + d] * hr;
+      ke += P[1 + d] * q[1 + d];
+    }
+    double e = q[D + 1] - ke;
+    if (GRAV) e -= q[0] * phi;
+    const double ib = 2 * (c.gamma - 1) * e * ir;  // 1/b = 2p/rho
+    P[0] = q[0];
+    P[D + 1] = fast_rcp(ib);
+    if (GRAV) {
+      P[D + 2] = 0.5 * phi;
+      P[D + 3] = 0.5 * ib;
+    }
+  }
+  // f/atanh f and atanh(f)/f in u = f^2 <= LM_U0: Chebyshev interpolants of degree 6 (3e-19 off)
+  ATM_DEV static double inv_series(double u) {
+#pragma clang fp contract(fast)
+    double s = -0.017268601586902934;
+    s = s * u + -0.02179015140718188;
+    s = s * u + -0.030194049011152555;
+    s = s * u + -0.04656084640141071;
+    s = s * u + -0.08888888888915485;
+    s = s * u + -0.33333333333333315;
+    return s * u + 1.0;
+  }
+  ATM_DEV static double series(double u) {
+#pragma clang fp contract(fast)
+    double s = 0.07930082527176203;
+    s = s * u + 0.09087619619304513;
+    s = s * u + 0.11111133605096339;
+    s = s * u + 0.1428571420685783;
+    s = s * u + 0.2000000000013155;
+    s = s * u + 0.33333333333333254;
+    return s * u + 1.0;
+  }
+  // sf: S/2 times row r of twice the flux's symmetric part; the fluctuation takes ta from momentum r
+  // of node a's sum and adds tb to what node b subtracts
+  template <int r>
+  ATM_DEV static void pair(double inv_gm1, const double* Pa, const double* Pb, double S, double* sf, double* ta,
+                           double* tb) {
+#pragma clang fp contract(fast)
+    const double ra = Pa[0], rb = Pb[0], ba = Pa[D + 1], bb = Pb[D + 1];
+    const double sr = ra + rb, sb = ba + bb;
+    const double i2 = fast_rcp(sr * sb);
+    const double isr = sb * i2, isb = sr * i2;
+    const double fr = (ra - rb) * isr, fb = (ba - bb) * isb;
+    const double ur = fr * fr, ub = fb * fb;
+    double Gr, Fb;
+    if (ur < LM_U0 && ub < LM_U0) {
+      Gr = inv_series(ur);
+      Fb = series(ub);
+    } else {
+      Gr = (ur < LM_U0) ? inv_series(ur) : 2 * fr / log(ra / rb);
+      Fb = (ub < LM_U0) ? series(ub) : log(ba / bb) / (2 * fb);
+    }
+    const double rl = sr * Gr;
+    const double pd = sr * isb;
+    double u[D], dot = Pa[1] * Pb[1];
+#pragma unroll
+    for (int d = 1; d < D; ++d) dot += Pa[1 + d] * Pb[1 + d];
+#pragma unroll
+    for (int d = 0; d < D; ++d) u[d] = Pa[1 + d] + Pb[1 + d];
+    double cc = Fb * isb * inv_gm1;
+    if (GRAV) cc += Pa[D + 2] + Pb[D + 2];
+    cc += 2 * dot;
+    const double su = S * u[r];
+    sf[0] = rl * su;
+#pragma unroll
+    for (int d = 0; d < D; ++d) sf[1 + d] = u[d] * sf[0];
+    sf[1 + r] += pd * S;
+    sf[D + 1] = su * (rl * cc + pd);
+    if (GRAV) {
+      const double t = S * (sb * rl * (Pa[D + 2] - Pb[D + 2]));
+      *ta = t * Pa[D + 3];
+      *tb = t * Pb[D + 3];
+    }
+  }
+};
 
 template <class L, int NQ>
 constexpr size_t fast_box_elem_doubles() {
-  return (size_t)box_planes<L>() * ipow(NQ, L::D) + box_xbuf<L, NQ>();
+  return (size_t)BoxEC<L>::NP * ipow(NQ, L::D) + box_xbuf<L, NQ>();
 }
 
 // FAST surface flux with the normal along the first momentum component
@@ -47,19 +137,17 @@ ATM_DEV void axis_fast_flux(const LawConst& c, const double* qm, double phim, do
                             double phip, double prefp, double* nf) {
   constexpr int D = L::D, Ns = L::Ns;
   constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
-  // the pressures keep the reference's rounding (fast_flux.hpp)
-  double pm, pfp, pp;
-  if constexpr (GRAV) {
-    pm = L::pressure(c, qm[0], qm + 1, qm[D + 1], phim);
-    pfp = L::pressure(c, qp[0], qp + 1, qp[D + 1], phip);
-    pp = SF == ATM_FLUX_ROE ? L::pressure(c, qp[0], qp + 1, qp[D + 1], phim) : pfp;
-  } else {
-    pm = L::pressure(c, qm[0], qm + 1, qm[D + 1]);
-    pp = pfp = L::pressure(c, qp[0], qp + 1, qp[D + 1]);
-  }
+  // the pressures keep the reference's rounding (fast_flux.hpp): the law's pressure() with its
+  // division rounded the same by fast_div
+  const double irm = fast_rcp(qm[0]), irp = fast_rcp(qp[0]);
+  const double gm1 = c.gamma - 1;
+  const double em = qm[D + 1] - fast_div(dotv<D>(qm + 1, qm + 1), 2 * qm[0], 0.5 * irm);
+  const double ep = qp[D + 1] - fast_div(dotv<D>(qp + 1, qp + 1), 2 * qp[0], 0.5 * irp);
+  const double pm = gm1 * (GRAV ? em - qm[0] * phim : em);
+  const double pfp = gm1 * (GRAV ? ep - qp[0] * phip : ep);
+  const double pp = GRAV && SF == ATM_FLUX_ROE ? gm1 * (ep - qp[0] * phim) : pfp;
   {
 #pragma clang fp contract(fast)
-    const double irm = fast_rcp(qm[0]), irp = fast_rcp(qp[0]);
     double um[D], up[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -137,8 +225,8 @@ struct BoxFaces {
       const int face = f / NFPF, fp = f - face * NFPF, r = face >> 1;
       const bool hi = face & 1;
       const int st = r == 0 ? 1 : (r == 1 ? NQ : NQ * NQ);
-      // face point -> node: the coordinates below direction r, then those above it
-      const int low = fp % st, ln0 = low + (fp - low) * NQ;
+      // face point (i, j) -> node: (0, i, j), (i, 0, j) or (i, j, 0)
+      const int ln0 = r == 0 ? fp * NQ : (r == 1 ? fp + (NQ * NQ - NQ) * (fp / NQ) : fp);
       const int ln = ln0 + (hi ? (NQ - 1) * st : 0);
       // a boundary face point reads its own node as the neighbour (every load unconditional)
       const uint32_t own = 8 * (e * Np + ln);
@@ -224,12 +312,12 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
                            int epw) {
 #pragma clang fp contract(fast)
   constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
-  using FE = FastEC<L::D, GRAV>;
-  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D), M = NQ / 2, NPL = box_planes<L>();
+  using EC = BoxEC<L>;
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D), M = NQ / 2, NPL = EC::NP;
   constexpr bool HALF = NQ % 2 == 0;  // the pairs at distance NQ/2 are taken by the lower half of each line
   constexpr int stride = (int)fast_box_elem_doubles<L, NQ>();
   static_assert(NPL >= Ns + (GRAV ? 1 : 0), "the surface term stages the state in the primitives' planes");
-  double* sS = lds;                // S_ab at [b + NQ a]
+  double* sS = lds;                // S_ab / 2 at [b + NQ a]
   double* siw = lds + NQ * NQ;     // 1 / w_a
   const int tid = threadIdx.x;
   const int el = tid / Np;
@@ -241,7 +329,7 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   double* sx = sP + NPL * Np;                     // [slot][s][node]
   for (int t = tid; t < NQ * NQ; t += blockDim.x) {
     const int b = t % NQ, a = t / NQ;
-    sS[t] = p.D[b + NQ * a] * p.bw[b] - p.D[a + NQ * b] * p.bw[a];
+    sS[t] = 0.5 * (p.D[b + NQ * a] * p.bw[b] - p.D[a + NQ * b] * p.bw[a]);
   }
   for (int t = tid; t < NQ; t += blockDim.x) siw[t] = 1 / p.bw[t];
   // every load of the node's data first and unconditionally (a lane past the last element reads
@@ -249,7 +337,7 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   const uint32_t e0 = active ? e : 0;
   const uint32_t node = 8 * (e0 * Np + ijk);
   const BoxElem<D>* rec = box_elem<D>(p, e0);
-  double q1[Ns], a1[NA], P1[FE::NP];
+  double q1[Ns], a1[NA], P1[NPL];
 #pragma unroll
   for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
   box_aux<L>(p, node, a1);
@@ -259,14 +347,10 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   using BF = BoxFaces<L, SF, NQ>;
   BF bf;
   bf.load(rec, ijk);
-  FE::prim(p.c, q1, a1, P1);
+  EC::prim(p.c, q1, GRAV ? a1[0] : 0.0, P1);
   if (active) {
 #pragma unroll
-    for (int k = 0; k < D + 2; ++k) sP[k * Np + ijk] = P1[k];
-    if constexpr (GRAV) {
-      sP[(D + 2) * Np + ijk] = P1[D + 3];
-      sP[(D + 3) * Np + ijk] = P1[D + 4];
-    }
+    for (int k = 0; k < NPL; ++k) sP[k * Np + ijk] = P1[k];
   }
   int idx[3];
   node_index<D>(ijk, NQ, idx);
@@ -286,10 +370,9 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   for (int s = 0; s < Ns; ++s) acc[s] = 0.0;
   if (active) L::sources(p.c, acc, q1, a1, all_dirs<L>(), false);
   __syncthreads();  // tables and primitives written
-#pragma unroll
-  for (int r = 0; r < D; ++r) {
+  for_dirs<0, D>([&](auto R) {
+    constexpr int r = decltype(R)::value, st = line_stride<NQ, r>();
     const int a = idx[r];
-    const int st = r == 0 ? 1 : (r == 1 ? NQ : NQ * NQ);
     const int lbase = ijk - a * st;
     double vol[Ns];
 #pragma unroll
@@ -303,33 +386,21 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
           if (HALF && m == M && a >= M) continue;
           const int b = a + m >= NQ ? a + m - NQ : a + m;
           const int ib = lbase + b * st;
-          double P2[FE::NP];
+          double P2[NPL];
 #pragma unroll
-          for (int k = 0; k < D + 2; ++k) P2[k] = sP[k * Np + ib];
-          P2[D + 2] = P2[1] * P2[1];
-#pragma unroll
-          for (int d = 1; d < D; ++d) P2[D + 2] += P2[1 + d] * P2[1 + d];
-          P2[D + 3] = GRAV ? sP[(D + 2) * Np + ib] : 0.0;
-          P2[D + 4] = GRAV ? sP[(D + 3) * Np + ib] : 0.0;
-          typename FE::Pair w;
-          FE::pair(p.c, inv_gm1, P1, P2, w);
-          const double S = sS[b + NQ * a];
-          // S times row r of the symmetric part of the flux
-          double sf[Ns];
-          const double su = S * w.u[r];
-          sf[0] = w.rho_log * su;
-#pragma unroll
-          for (int d = 0; d < D; ++d) sf[1 + d] = w.u[d] * sf[0];
-          sf[1 + r] += w.pd * S;
-          sf[D + 1] = su * w.ecoef;
+          for (int k = 0; k < NPL; ++k) P2[k] = sP[k * Np + ib];
+          double sf[Ns], ta, tb;
+          EC::template pair<r>(inv_gm1, P1, P2, sS[b + NQ * a], sf, &ta, &tb);
 #pragma unroll
           for (int s = 0; s < Ns; ++s) vol[s] += sf[s];
-          if (GRAV) vol[1 + r] -= S * w.fla;
+          if (GRAV) {
+            vol[1 + r] -= ta;
+            sf[1 + r] += tb;
+          }
           // the partner's share, which it subtracts
           const bool hs = HALF && m == M;
           double* slot = sx + (m - m0) * Ns * Np + (hs ? half_pos(r, b) : ib);
           const int xs = hs ? Np / 2 : Np;
-          if (GRAV) sf[1 + r] -= S * w.flb;
 #pragma unroll
           for (int s = 0; s < Ns; ++s) slot[s * xs] = sf[s];
         }
@@ -353,14 +424,14 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
       acc[s] += gw * vol[s];
       asm("" : "+v"(acc[s]));  // summed here: the compiler would keep every direction's vol until the end
     }
-  }
+  });
   // Surface term: no thread reads a partner's primitives any more, so the state and geopotential are
   // staged by node in their planes; the face points read their own side there, the update the state.
   double* sQ = sP;
   if (active) {
 #pragma unroll
     for (int s = 0; s < Ns; ++s) sQ[s * Np + ijk] = ldo(p, q, s, node);
-    if constexpr (GRAV) sQ[Ns * Np + ijk] = P1[D + 3];
+    if constexpr (GRAV) sQ[Ns * Np + ijk] = 2 * P1[D + 2];  // = aux[0]
   }
   __syncthreads();  // every thread has consumed its exchange slots
   if (active) bf.run(p, rec, e, ijk, q, sx, sQ, siw[0]);

@@ -17,31 +17,36 @@
 
 namespace atm {
 
-// 1/x for positive normal x: the hardware reciprocal refined by two Newton
-// steps (within about one ulp), about a third of an IEEE division.
+// 1/x for positive normal x: the hardware reciprocal (24 bits) refined by one third-order step
+// (at most half an ulp off in 2 million quotients, as two Newton steps are), about a third of an
+// IEEE division.
 __device__ __forceinline__ double fast_rcp(double x) {
 #pragma clang fp contract(fast)
-  double r = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-x, r, 1.0);
-  return fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 
 // sqrt(x) for positive normal x: the hardware reciprocal square root y refined by
-// two coupled Newton (Goldschmidt) steps on g = x*y ~ sqrt(x) and h = y/2 ~
-// 1/(2 sqrt(x)), then one residual correction g + h (x - g^2) (within about one ulp).
+// a coupled Newton (Goldschmidt) step on g = x*y ~ sqrt(x) and h = y/2 ~
+// 1/(2 sqrt(x)), then one residual correction g + h (x - g^2), which doubles the
+// digits once more (at most half an ulp off in 2 million roots).
 __device__ __forceinline__ double fast_sqrt(double x) {
 #pragma clang fp contract(fast)
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const double r = fma(-g, h, 0.5);
-    g = fma(g, r, g);
-    h = fma(h, r, h);
-  }
+  const double r = fma(-g, h, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
   return fma(fma(-g, g, x), h, g);
+}
+
+// a/x from ix = fast_rcp(x): the quotient with one residual correction, which rounds as an IEEE
+// division does
+__device__ __forceinline__ double fast_div(double a, double x, double ix) {
+#pragma clang fp contract(fast)
+  const double q = a * ix;
+  return fma(fma(-x, q, a), ix, q);
 }
 
 template <class L, int SF>
