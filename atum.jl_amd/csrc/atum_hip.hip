@@ -1469,7 +1469,7 @@ int atm_dg_create(atm_ctx* ctx, const atm_dg_desc* d, atm_dg** out) {
       (rc = upload_copy(dg, d->faceMJ, (size_t)NF, &p.faceMJ)) ||
       (rc = upload_copy(dg, d->normal, (size_t)d->dim * NF, &p.normal)) ||
       (rc = upload_copy(dg, d->faceix_p, (size_t)NF, &p.faceix_p)) ||
-      (rc = upload_copy(dg, d->bctag, (size_t)2 * d->dim * d->K, &p.bctag)) || (rc = dg_box(dg, d, nullptr))) {
+      (rc = upload_copy(dg, d->bctag, (size_t)2 * d->dim * d->K, &p.bctag)) || (rc = dg_box(dg, d))) {
     atm_dg_destroy(dg);
     return rc;
   }

@@ -145,55 +145,34 @@ void lgl_weights(int Nq, double* w) {
 
 namespace atm {
 
-int dg_box(atm_dg* dg, const atm_dg_desc* d, const double* w_host) {
-  DevDG& p = dg->dev;
-  if (p.K < 1 || dg->Ns * dg->Ntot >= BOX_MAX_STATE) return ATM_OK;
-  const Resolved r = resolve_box(d, dg->Nq);
-  atm_ctx* ctx = dg->ctx;
-  if (!r.fn || r.lds > ctx->max_lds) return ATM_OK;
-  const int dim = dg->dim, Nq = dg->Nq, Np = dg->Np;
-  std::vector<double> tab((size_t)Nq + Np + p.Nfpf);
-  double* w = tab.data();
-  double* wp = w + Nq;
-  double* wf = wp + Np;
-  if (w_host) std::memcpy(w, w_host, sizeof(double) * Nq);
-  else lgl_weights(Nq, w);
-  for (int t = 0; t < Np + p.Nfpf; ++t) {
+std::vector<double> box_tables(int dim, int Nq, const double* w) {
+  const int Np = ipow(Nq, dim), Nfpf = Np / Nq;
+  std::vector<double> tab((size_t)Nq + Np + Nfpf);
+  std::memcpy(tab.data(), w, sizeof(double) * Nq);
+  for (int t = 0; t < Np + Nfpf; ++t) {
     int rem = t < Np ? t : t - Np;
     double v = 1.0;
     for (int i = 0; i < (t < Np ? dim : dim - 1); ++i) {
       v = v * w[rem % Nq];
       rem /= Nq;
     }
-    (t < Np ? wp[t] : wf[t - Np]) = v;
+    tab[(size_t)Nq + t] = v;
   }
-  const size_t bytes = (size_t)(2 * dim + 1) * sizeof(double) + (size_t)2 * dim * sizeof(int32_t);
-  const size_t head = (tab.size() * sizeof(double) + sizeof(int32_t) + 255) / 256 * 256;
-  void* mem = nullptr;
-  HIPCHK(ctx, hipMalloc(&mem, head + bytes * (size_t)p.K));
-  double* dtab = static_cast<double*>(mem);
-  int32_t* bad = reinterpret_cast<int32_t*>(dtab + tab.size());
-  char* rec = static_cast<char*>(mem) + head;
-  std::vector<char> init(tab.size() * sizeof(double) + sizeof(int32_t), 0);  // weights, then the flag
-  std::memcpy(init.data(), tab.data(), tab.size() * sizeof(double));
-  hipStream_t s = stream_of(ctx);
-  int32_t host_bad = 1;
-  hipError_t e = hipMemcpy(mem, init.data(), init.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(box_detect_kernel, dim3(p.K < 65536 ? p.K : 65536), dim3(256), 0, s, p, dim, dtab + Nq,
-                       dtab + Nq + Np, rec, (int)bytes, bad);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = hipMemcpy(&host_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost);
-  if (e != hipSuccess || host_bad) {
-    hipFree(mem);
-    return e == hipSuccess ? ATM_OK : hipfail(ctx, e, "box element detection");
-  }
-  dg->allocs.push_back(mem);
-  dg->dev_bytes += head + bytes * (size_t)p.K;
+  return tab;
+}
+
+size_t box_elem_bytes(int dim) { return (size_t)(2 * dim + 1) * sizeof(double) + (size_t)2 * dim * sizeof(int32_t); }
+
+bool box_kernels(const atm_dg* dg, const atm_dg_desc* d, Resolved* r) {
+  if (dg->dev.K < 1 || dg->Ns * dg->Ntot >= BOX_MAX_STATE) return false;
+  *r = resolve_box(d, dg->Nq);
+  return r->fn && r->lds <= dg->ctx->max_lds;
+}
+
+void dg_use_box(atm_dg* dg, const Resolved& r, const void* rec, const double* tab) {
+  DevDG& p = dg->dev;
   p.box = rec;
-  p.bw = dtab;
+  p.bw = tab;
   dg->fn = r.fn;
   dg->bfn = r.bfn;
   dg->mbfn = r.mbfn;
@@ -204,6 +183,42 @@ int dg_box(atm_dg* dg, const atm_dg_desc* d, const double* w_host) {
   dg->max_threads = r.max_threads;
   p.epw = r.epw;
   p.lds = (int)r.lds;
+}
+
+int dg_box(atm_dg* dg, const atm_dg_desc* d) {
+  DevDG& p = dg->dev;
+  Resolved r;
+  if (!box_kernels(dg, d, &r)) return ATM_OK;
+  atm_ctx* ctx = dg->ctx;
+  const int dim = dg->dim, Nq = dg->Nq, Np = dg->Np;
+  double w[8];
+  lgl_weights(Nq, w);
+  std::vector<double> tab = box_tables(dim, Nq, w);
+  tab.push_back(0.0);  // the flag that box_detect_kernel raises
+  const size_t bytes = box_elem_bytes(dim);
+  const size_t head = (tab.size() * sizeof(double) + 255) / 256 * 256;
+  void* mem = nullptr;
+  HIPCHK(ctx, hipMalloc(&mem, head + bytes * (size_t)p.K));
+  double* dtab = static_cast<double*>(mem);
+  int32_t* bad = reinterpret_cast<int32_t*>(dtab + tab.size() - 1);
+  char* rec = static_cast<char*>(mem) + head;
+  hipStream_t s = stream_of(ctx);
+  int32_t host_bad = 1;
+  hipError_t e = hipMemcpy(mem, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(box_detect_kernel, dim3(p.K < 65536 ? p.K : 65536), dim3(Np > 128 ? 256 : 64), 0, s, p, dim,
+                       dtab + Nq, dtab + Nq + Np, rec, (int)bytes, bad);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = hipMemcpy(&host_bad, bad, sizeof(int32_t), hipMemcpyDeviceToHost);
+  if (e != hipSuccess || host_bad) {
+    hipFree(mem);
+    return e == hipSuccess ? ATM_OK : hipfail(ctx, e, "box element detection");
+  }
+  dg->allocs.push_back(mem);
+  dg->dev_bytes += head + bytes * (size_t)p.K;
+  dg_use_box(dg, r, rec, dtab);
   return ATM_OK;
 }
 

@@ -72,7 +72,7 @@ ATM_DEV void box_epilogue(const DevDG& p, uint32_t off, const double* q1, const 
   }
 }
 
-constexpr int ipow(int b, int n) { return n == 0 ? 1 : b * ipow(b, n - 1); }
+__host__ __device__ constexpr int ipow(int b, int n) { return n == 0 ? 1 : b * ipow(b, n - 1); }
 
 // The direction mask of an operator of all directions
 template <class L>

@@ -5,12 +5,15 @@
 // One thread per volume node computes the node coordinates, MJ = w_i w_j w_k J,
 // MJI = 1/MJ and the affine metric g = diag(2/h); one thread per face point
 // computes the face tables (neighbour node, boundary tag), faceMJ and the unit
-// normal.  Every value is formed with the same operations in the same order as
-// the host builder (atum_hip/grid.py), so both produce identical bits.
+// normal; one thread per element writes the compact record of box.hpp, whose
+// values reproduce those arrays.  Every value is formed with the same operations
+// in the same order as the host builder (atum_hip/grid.py), so both produce
+// identical bits.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
 
+#include "box.hpp"
 #include "handles.hpp"
 
 namespace {
@@ -129,6 +132,41 @@ __global__ void brick_face_kernel(BrickGeo b, int64_t* __restrict__ faceix_p, do
   }
 }
 
+template <int D>
+__global__ void brick_box_kernel(BrickGeo b, BoxElem<D>* __restrict__ rec) {
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < b.K; e += (int64_t)gridDim.x * blockDim.x) {
+    int em[3];
+    elem_multi(b, e, em);
+    BoxElem<D> x;
+    double h[D];
+    x.J = 1.0;
+    for (int d = 0; d < D; ++d) {
+      h[d] = b.coords[d][em[d] + 1] - b.coords[d][em[d]];
+      x.g[d] = 2 / h[d];
+      x.J = d == 0 ? h[d] / 2 : x.J * (h[d] / 2);
+    }
+    for (int r = 0; r < D; ++r) {
+      x.fJ[r] = 1.0;
+      for (int d = 0; d < D; ++d)
+        if (d != r) x.fJ[r] = x.fJ[r] * (h[d] / 2);
+      for (int side = 0; side < 2; ++side) {
+        int nb[3] = {em[0], em[1], em[2]};
+        nb[r] += side == 0 ? -1 : 1;
+        const bool out = nb[r] < 0 || nb[r] >= b.Kd[r];
+        if (out) nb[r] = side == 0 ? b.Kd[r] - 1 : 0;
+        x.nb[2 * r + side] = out && !b.periodic[r] ? -(2 * r + side + 1) : (int32_t)elem_id(b, nb);
+      }
+    }
+    rec[e] = x;
+  }
+}
+
+void launch_brick_box(int blocks, hipStream_t s, const BrickGeo& b, void* rec) {
+  if (b.dim == 1) hipLaunchKernelGGL(brick_box_kernel<1>, dim3(blocks), dim3(256), 0, s, b, (BoxElem<1>*)rec);
+  if (b.dim == 2) hipLaunchKernelGGL(brick_box_kernel<2>, dim3(blocks), dim3(256), 0, s, b, (BoxElem<2>*)rec);
+  if (b.dim == 3) hipLaunchKernelGGL(brick_box_kernel<3>, dim3(blocks), dim3(256), 0, s, b, (BoxElem<3>*)rec);
+}
+
 inline int grid_blocks(int64_t n) {
   int64_t g = (n + 255) / 256;
   return (int)(g > 65535 * 16 ? 65535 * 16 : (g < 1 ? 1 : g));
@@ -170,32 +208,52 @@ int atm_dg_create_brick(atm_ctx* ctx, const atm_dg_desc* d, const atm_brick_desc
   b.K = K;
   b.Ntot = Ntot;
   b.NF = NF;
-  const double* cdev[3] = {nullptr, nullptr, nullptr};
+  // one upload: vertex coordinates, LGL nodes, D, and the weights with their products
+  std::vector<double> tab;
+  size_t at[3] = {0, 0, 0};
+  for (int i = 0; i < dim; ++i) {
+    at[i] = tab.size();
+    tab.insert(tab.end(), bd->coords[i], bd->coords[i] + bd->Kd[i] + 1);
+  }
+  const size_t at_xi = tab.size();
+  tab.insert(tab.end(), bd->xi, bd->xi + Nq);
+  const size_t at_D = tab.size();
+  tab.insert(tab.end(), d->D, d->D + (size_t)Nq * Nq);
+  const size_t at_w = tab.size();
+  const std::vector<double> wt = box_tables(dim, Nq, bd->w);
+  tab.insert(tab.end(), wt.begin(), wt.end());
+  const double* dtab = nullptr;
+  rc = upload_copy(dg, tab.data(), tab.size(), &dtab);
+  if (rc == ATM_OK) {
+    b.xi = dtab + at_xi;
+    b.w = dtab + at_w;
+    p.D = dtab + at_D;
+  }
+  Resolved box;
+  const bool use_box = box_kernels(dg, d, &box);
   void *pts = nullptr, *g = nullptr, *MJ = nullptr, *MJI = nullptr, *fMJ = nullptr, *nrm = nullptr, *fxp = nullptr,
-       *tag = nullptr;
-  for (int i = 0; i < dim && rc == ATM_OK; ++i) rc = upload_copy(dg, bd->coords[i], (size_t)bd->Kd[i] + 1, &cdev[i]);
-  if (rc == ATM_OK) rc = upload_copy(dg, bd->xi, (size_t)Nq, &b.xi);
-  if (rc == ATM_OK) rc = upload_copy(dg, bd->w, (size_t)Nq, &b.w);
-  if (rc == ATM_OK) rc = upload_copy(dg, d->D, (size_t)Nq * Nq, &p.D);
+       *tag = nullptr, *rec = nullptr;
   const size_t S = sizeof(double);
   if (rc == ATM_OK && Ntot > 0 &&
       ((rc = dg_alloc(dg, (size_t)dim * Ntot * S, &pts)) || (rc = dg_alloc(dg, (size_t)dim * dim * Ntot * S, &g)) ||
        (rc = dg_alloc(dg, (size_t)Ntot * S, &MJ)) || (rc = dg_alloc(dg, (size_t)Ntot * S, &MJI)) ||
        (rc = dg_alloc(dg, (size_t)NF * S, &fMJ)) || (rc = dg_alloc(dg, (size_t)dim * NF * S, &nrm)) ||
        (rc = dg_alloc(dg, (size_t)NF * sizeof(int64_t), &fxp)) ||
-       (rc = dg_alloc(dg, (size_t)2 * dim * K * sizeof(int32_t), &tag)))) {
+       (rc = dg_alloc(dg, (size_t)2 * dim * K * sizeof(int32_t), &tag)) ||
+       (use_box && (rc = dg_alloc(dg, box_elem_bytes(dim) * (size_t)K, &rec))))) {
   }
   if (rc) {
     atm_dg_destroy(dg);
     return rc;
   }
-  for (int i = 0; i < 3; ++i) b.coords[i] = cdev[i];
+  for (int i = 0; i < 3; ++i) b.coords[i] = dtab + at[i];
   if (Ntot > 0) {
     hipStream_t s = stream_of(ctx);
     hipLaunchKernelGGL(brick_volume_kernel, dim3(grid_blocks(Ntot)), dim3(256), 0, s, b, (double*)pts, (double*)g,
                        (double*)MJ, (double*)MJI);
     hipLaunchKernelGGL(brick_face_kernel, dim3(grid_blocks(NF)), dim3(256), 0, s, b, (int64_t*)fxp, (double*)fMJ,
                        (double*)nrm, (int32_t*)tag);
+    if (use_box) launch_brick_box(grid_blocks(K), s, b, rec);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
@@ -211,10 +269,7 @@ int atm_dg_create_brick(atm_ctx* ctx, const atm_dg_desc* d, const atm_brick_desc
   p.normal = (const double*)nrm;
   p.faceix_p = (const int64_t*)fxp;
   p.bctag = (const int32_t*)tag;
-  if ((rc = dg_box(dg, d, bd->w))) {
-    atm_dg_destroy(dg);
-    return rc;
-  }
+  if (use_box) dg_use_box(dg, box, rec, dtab + at_w);
   *out = dg;
   return ATM_OK;
 }

@@ -93,9 +93,15 @@ int dg_prepare(atm_ctx* ctx, const atm_dg_desc* d, atm_dg** out);
 Resolved resolve_box(const atm_dg_desc* d, int Nq);
 
 // Looks whether the operator's elements are all boxes, its geometry arrays being on the device;
-// if so, and there are kernels for it, builds the compact geometry and selects them.  w_host: the LGL
-// weights the geometry was built with (null: computed here).
-int dg_box(atm_dg* dg, const atm_dg_desc* d, const double* w_host);
+// if so, and there are kernels for it, builds the compact geometry and selects them.
+int dg_box(atm_dg* dg, const atm_dg_desc* d);
+
+// The parts of it for an operator that is known to consist of boxes: whether there are kernels, the
+// weight tables from the LGL weights, a record's size, and the selection.
+bool box_kernels(const atm_dg* dg, const atm_dg_desc* d, Resolved* r);
+std::vector<double> box_tables(int dim, int Nq, const double* w);
+size_t box_elem_bytes(int dim);
+void dg_use_box(atm_dg* dg, const Resolved& r, const void* rec, const double* tab);
 
 // The linear operator a banded factorisation was built from.
 atm_dg* banded_lin(const atm_banded* b);
