@@ -227,10 +227,13 @@ Resolved resolve_box_weak_euler_gravity(int dim, int mask, int Nq);
 Resolved resolve_box_weak_linear(int dim, int mask, int Nq);
 Resolved resolve_box_weak_shallow_water(int dim, int mask, int Nq);
 
-Resolved resolve_box_fast_euler_roe(int dim, int Nq);
-Resolved resolve_box_fast_euler_rusanov(int dim, int Nq);
-Resolved resolve_box_fast_euler_gravity_roe(int dim, int Nq);
-Resolved resolve_box_fast_euler_gravity_rusanov(int dim, int Nq);
+#define ATM_BOX_EC(FORM, LAW) \
+  Resolved resolve_box_##FORM##_##LAW##_roe(int dim, int Nq); \
+  Resolved resolve_box_##FORM##_##LAW##_rusanov(int dim, int Nq);
+ATM_BOX_EC(fast, euler)
+ATM_BOX_EC(fast, euler_gravity)
+ATM_BOX_EC(fd, euler)
+ATM_BOX_EC(fd, euler_gravity)
 
 // Kernels for an operator whose elements are all boxes (fn == nullptr: the general ones)
 Resolved resolve_box(const atm_dg_desc* d, int Nq) {
@@ -243,14 +246,16 @@ Resolved resolve_box(const atm_dg_desc* d, int Nq) {
       default: break;
     }
   if (d->volume_form == ATM_FORM_FLUX_DIFFERENCING && d->volume_flux == ATM_FLUX_EC &&
-      d->precision == ATM_PRECISION_FAST && d->dirmask == (1 << d->dim) - 1) {
-    const bool roe = d->surface_flux == ATM_FLUX_ROE;
-    if (roe || d->surface_flux == ATM_FLUX_RUSANOV) {
-      if (d->law == ATM_LAW_EULER)
-        return roe ? resolve_box_fast_euler_roe(d->dim, Nq) : resolve_box_fast_euler_rusanov(d->dim, Nq);
-      if (d->law == ATM_LAW_EULER_GRAVITY)
-        return roe ? resolve_box_fast_euler_gravity_roe(d->dim, Nq) : resolve_box_fast_euler_gravity_rusanov(d->dim, Nq);
+      d->fd_kernel == ATM_FD_PER_DIR && d->dirmask == (1 << d->dim) - 1 &&
+      (d->surface_flux == ATM_FLUX_ROE || d->surface_flux == ATM_FLUX_RUSANOV)) {
+    const bool roe = d->surface_flux == ATM_FLUX_ROE, grav = d->law == ATM_LAW_EULER_GRAVITY;
+    if (!grav && d->law != ATM_LAW_EULER) return Resolved{nullptr, 0, 0, nullptr, 1};
+    if (d->precision == ATM_PRECISION_FAST && d->dim >= 2) {  // FAST precision has no 1-D kernels of its own
+      if (grav) return roe ? resolve_box_fast_euler_gravity_roe(d->dim, Nq) : resolve_box_fast_euler_gravity_rusanov(d->dim, Nq);
+      return roe ? resolve_box_fast_euler_roe(d->dim, Nq) : resolve_box_fast_euler_rusanov(d->dim, Nq);
     }
+    if (grav) return roe ? resolve_box_fd_euler_gravity_roe(d->dim, Nq) : resolve_box_fd_euler_gravity_rusanov(d->dim, Nq);
+    return roe ? resolve_box_fd_euler_roe(d->dim, Nq) : resolve_box_fd_euler_rusanov(d->dim, Nq);
   }
   return Resolved{nullptr, 0, 0, nullptr, 1};
 }

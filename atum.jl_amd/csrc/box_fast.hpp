@@ -14,6 +14,7 @@
 #pragma once
 #include "box.hpp"
 #include "fd_fast.hpp"
+#include "log_mean.hpp"
 
 namespace atm {
 
@@ -61,54 +62,6 @@ struct BoxEC {
       P[D + 3] = 0.5 * ib;
     }
   }
-  // f/atanh f and atanh(f)/f in u = f^2 <= LM_U0: Chebyshev interpolants of degree 6 (3e-19 off)
-  ATM_DEV static double inv_series(double u) {
-#pragma clang fp contract(fast)
-    double s = u * -0.017268601586902934 + -0.02179015140718188;
-    s = s * u + -0.030194049011152555;
-    s = s * u + -0.04656084640141071;
-    s = s * u + -0.08888888888915485;
-    s = s * u + -0.33333333333333315;
-    return s * u + 1.0;
-  }
-  ATM_DEV static double series(double u) {
-#pragma clang fp contract(fast)
-    double s = u * 0.07930082527176203 + 0.09087619619304513;
-    s = s * u + 0.11111133605096339;
-    s = s * u + 0.1428571420685783;
-    s = s * u + 0.2000000000013155;
-    s = s * u + 0.33333333333333254;
-    return s * u + 1.0;
-  }
-  // log z for z outside [0.8, 1.2]: 2 atanh((m-1)/(m+1)) + k log 2, z = 2^k m, m in [sqrt 1/2, sqrt 2)
-  // (at most 2 ulps off, 0.41 rms; the library's log takes 99 instructions and more registers than the
-  // rest of the kernel, this one 30).  Zero, infinity, negatives and NaN as log.
-  ATM_DEV static double log_ratio(double z) {
-#pragma clang fp contract(fast)
-    double m = __builtin_amdgcn_frexp_mant(z);
-    int k = __builtin_amdgcn_frexp_exp(z);
-    const bool lo = m < 0.70710678118654752;
-    m = lo ? 2 * m : m;
-    k = lo ? k - 1 : k;
-    const double d = m - 1, s = m + 1;
-    const double f = fast_div(d, s, fast_rcp(s));
-    const double u = f * f, t = 2 * f, kd = k;
-    double q = u * 0.07404933786156531 + 0.0765625655736915;
-    q = q * u + 0.09091816120808513;
-    q = q * u + 0.11111098523202137;
-    q = q * u + 0.1428571438036914;
-    q = q * u + 0.19999999999650955;
-    q = q * u + 0.33333333333333826;
-    const double r = kd * 0.693147180559663 + ((kd * 2.8235290563031577e-13 + t) + t * u * q);
-    if (z > 0 && z < HUGE_VAL) return r;
-    return z == 0 ? -HUGE_VAL : (z > 0 ? z : __builtin_nan(""));
-  }
-  // atanh(f)/f = log(a/b) / 2f for a and b that far apart, f = (a-b)/(a+b)
-  ATM_DEV static double far_ratio(double a, double b) {
-    const double d = a - b, s = a + b, z = fast_div(a, b, fast_rcp(b)), h = 2 * fast_div(d, s, fast_rcp(s));
-    const double l = log_ratio(z);
-    return fast_div(l, h, fast_rcp(h));
-  }
   // sf: S/2 times row r of twice the flux's symmetric part; the fluctuation takes ta from momentum r
   // of node a's sum and adds tb to what node b subtracts
   template <int r>
@@ -122,12 +75,12 @@ struct BoxEC {
     const double fr = (ra - rb) * isr, fb = (ba - bb) * isb;
     const double ur = fr * fr, ub = fb * fb;
     double Gr, Fb;
-    if (ur < LM_U0 && ub < LM_U0) {
-      Gr = inv_series(ur);
-      Fb = series(ub);
+    if (ur < LM_U && ub < LM_U) {
+      Gr = lm_inverse(ur);
+      Fb = lm_direct(ub);
     } else {
-      Gr = (ur < LM_U0) ? inv_series(ur) : fast_rcp(far_ratio(ra, rb));
-      Fb = (ub < LM_U0) ? series(ub) : far_ratio(ba, bb);
+      Gr = lm_g(ra, rb, ur);
+      Fb = lm_f(ba, bb, ub);
     }
     const double rl = sr * Gr;
     const double pd = sr * isb;

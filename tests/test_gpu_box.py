@@ -112,6 +112,22 @@ FAST = [("euler", 2, (4, 3), dict(bc="prescribed", periodic=False)), ("euler", 2
         ("euler_gravity", 3, (3, 2, 2), dict(bc="copy", periodic=(True, False, False), ordering="stacked"))]
 
 
+FD = FAST + [("euler", 1, (7,), dict(bc="prescribed", periodic=False)),
+             ("euler_gravity", 1, (5,), dict(bc="reflect", periodic=False))]
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("sflux", ["roe", "rusanov"])
+@pytest.mark.parametrize("law,dim,Kd,kw", FD, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(FD)])
+def test_reference_order_box_kernels_against_the_general_ones(law, dim, Kd, kw, sflux, N):
+    """The same order of the sums with another form of the logarithmic means: each form is within 1e-12
+    of the oracle's tendency (relative max-norm, tests/test_gpu_parity.py)."""
+    box, general, q0 = pair(law, dim, N, Kd, form="ec", sflux=sflux, seed=20 + N, **kw)
+    assert device_bytes(box) > device_bytes(general)
+    a, b = tendencies(box, general, q0)
+    assert np.abs(a - b).max() <= 2e-12 * np.abs(b).max()
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("sflux", ["roe", "rusanov"])
 @pytest.mark.parametrize("law,dim,Kd,kw", FAST, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(FAST)])
