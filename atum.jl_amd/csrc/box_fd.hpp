@@ -4,9 +4,12 @@
 // The sums keep the reference's order, every product and sum rounded; with a diagonal metric only row
 // r of the two-point flux enters direction r, a third of the products.  Quotients and square roots are
 // fast_div and fast_sqrt, which round as IEEE's do, by reciprocals that the pair's or node's quotients
-// share; the logarithm of the logarithmic means is lm_logavg's (a seventh of the instructions of
+// share; the logarithm of the logarithmic means is lm_logavg2's (a seventh of the instructions of
 // the library's, and as close).  Every value equals the general kernels' but for the last bit of
 // that logarithm.
+//
+// Bound by FP64 instructions: about 165 for an ordered pair and 290 for a face.  Against the general
+// kernels, per stage: bubble 12^3 N = 4 (Roe) 78 -> 38 us, vortex 8^2 N = 4 15.5 -> 8.1 us.
 #pragma once
 #include "box.hpp"
 #include "log_mean.hpp"
@@ -126,15 +129,17 @@ struct BoxPairEC {
   ATM_DEV static void pair(double gm1x2, const double* P1, double ib2, const double* P2, double* F) {
     const double r1 = P1[0], r2 = P2[0], b1 = P1[D + 1], b2 = P2[D + 1];
     const double sr = r1 + r2, sb = b1 + b2;
-    const double rho_log = lm_logavg(r1, r2, fast_rcp(r2)), b_log = lm_logavg(b1, b2, fast_rcp(b2));
+    double rho_log, b_log;
+    lm_logavg2(r1, r2, b1, b2, &rho_log, &b_log);
+    const double den = gm1x2 * b_log, ii = rcp_div(sb * den);
     double u[D], frho[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       u[d] = avg(P1[1 + d], P2[1 + d]);
       frho[d] = u[d] * rho_log;
     }
-    const double pd = fast_div(sr / 2, sb, fast_rcp(sb));
-    double cc = fast_rcp(gm1x2 * b_log) - avg(P1[D + 2], P2[D + 2]) / 2;
+    const double pd = fast_div(sr / 2, sb, den * ii);
+    double cc = fast_div(1.0, den, sb * ii) - avg(P1[D + 2], P2[D + 2]) / 2;
     if (GRAV) cc = cc + avg(P1[D + 3], P2[D + 3]);
     double mv = 0;
 #pragma unroll
@@ -148,6 +153,77 @@ struct BoxPairEC {
   }
 };
 
+// Direction r's volume sum of one node, from -0.0 on with its sources, n ascending
+template <class L, int NQ, int r>
+ATM_DEV void fd_box_dir(const DevDG& p, const double* sD, const double* sP, int ijk, int id, double g, double MJn,
+                        double MJIn, const double* q1, const double* a1, const double* P1, double* dl) {
+  using PF = BoxPairEC<L>;
+  constexpr int Ns = L::Ns, Np = ipow(NQ, L::D), NP = PF::NP, st = line_stride<NQ, r>();
+  const double gm1x2 = 2 * (p.c.gamma - 1);
+  const double ib2 = fast_rcp(2 * P1[L::D + 1]);
+  const double* line = sP + ijk - id * st;
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) dl[s] = -0.0;
+  L::sources(p.c, dl, q1, a1, 1 << r, false);
+  const double lgi = MJn * g;
+  // not unrolled: two pairs at once take 200 registers and gain nothing (the branch to the far
+  // logarithms keeps them apart)
+#pragma unroll 1
+  for (int n = 0; n < NQ; ++n) {
+    double P2[NP], F[Ns];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) P2[k] = line[k * Np + n * st];
+    PF::template pair<r>(gm1x2, P1, ib2, P2, F);
+    const double ci = MJIn * sD[id + NQ * n] * lgi;
+    const double lgn = line[NP * Np + n * st] * g;
+    const double cn = MJIn * sD[n + NQ * id];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) {
+      dl[s] -= ci * F[s];
+      dl[s] += F[s] * lgn * cn;
+    }
+  }
+}
+
+// Byte offset of the node across the face that a node of line position ir lies on in direction r (its own
+// at a boundary, so that the loads there need no branch)
+template <int NQ, int D>
+ATM_DEV uint32_t across(int r, bool hi, int nb, uint32_t e, int ijk) {
+  const int span = (NQ - 1) * (r == 0 ? 1 : (r == 1 ? NQ : NQ * NQ));
+  return 8 * (nb >= 0 ? (uint32_t)nb * ipow(NQ, D) + ijk + (hi ? -span : span) : e * ipow(NQ, D) + ijk);
+}
+
+// What the face of direction r (the outward normal sg e_r) takes from the node, qp and ap the state and
+// aux across it
+template <class L, int SF, int r>
+ATM_DEV void fd_box_face(const DevDG& p, int nb, double sg, const double* q1, const double* a1, double* qp, double* ap,
+                         double fMJ, double MJIn, double* sf) {
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA;
+  if (nb < 0) {
+    double n[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) n[d] = d == r ? sg : 0.0;
+    boundarystate<L>(p.c, n, q1, -nb, qp);
+#pragma unroll
+    for (int s = 0; s < NA; ++s) ap[s] = a1[s];
+  }
+  double nf[Ns];
+  axis_ref_flux<L, SF, r>(p.c, sg, q1, a1, qp, ap, nf);
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) sf[s] = fMJ * nf[s] * MJIn;
+}
+
+// The weights' product on a face of direction r, in the order faceMJ has it
+template <int D>
+ATM_DEV double face_weight(const double* sw, const int idx[3], int r) {
+  double wf = 1.0;
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d != r) wf = wf * sw[idx[d]];
+  return wf;
+}
+
+// One thread per node: the directions one after the other.
 template <class L, int NQ, int SF>
 ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
                          double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
@@ -170,11 +246,11 @@ ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double*
   const uint32_t node = 8 * (e0 * Np + ijk);
   int idx[3];
   node_index<D>(ijk, NQ, idx);
-  const BoxElem<D> b = *box_elem<D>(p, e0);
+  const BoxElem<D>* rec = box_elem<D>(p, e0);
 #pragma unroll
   for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
   box_aux<L>(p, node, a1);
-  const double MJn = p.bw[NQ + ijk] * b.J;
+  const double MJn = p.bw[NQ + ijk] * rec->J;
   PF::prim(p.c, q1, a1, P1);
   if (active) {
 #pragma unroll
@@ -184,70 +260,161 @@ ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double*
   __syncthreads();
   if (!active) return;
   const double MJIn = fast_rcp(MJn);
-  const double gm1x2 = 2 * (p.c.gamma - 1);
-  const double ib2 = fast_rcp(2 * P1[D + 1]);
   double acc[Ns];
 #pragma unroll
   for (int s = 0; s < Ns; ++s) acc[s] = assign ? 0.0 : alpha * ldo(p, dq, s, node);
   for_dirs<0, D>([&](auto R) {
-    constexpr int r = decltype(R)::value, st = line_stride<NQ, r>();
-    const int id = idx[r];
-    const double* line = sP + ijk - id * st;
+    constexpr int r = decltype(R)::value;
     double dl[Ns];
+    fd_box_dir<L, NQ, r>(p, sD, sP, ijk, idx[r], rec->g[r], MJn, MJIn, q1, a1, P1, dl);
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) dl[s] = -0.0;
-    L::sources(p.c, dl, q1, a1, 1 << r, false);
-    const double lgi = MJn * b.g[r];
-#pragma unroll 1
-    for (int n = 0; n < NQ; ++n) {
-      double P2[NP], F[Ns];
-#pragma unroll
-      for (int k = 0; k < NP; ++k) P2[k] = line[k * Np + n * st];
-      PF::template pair<r>(gm1x2, P1, ib2, P2, F);
-      const double ci = MJIn * sD[id + NQ * n] * lgi;
-      const double lgn = line[NP * Np + n * st] * b.g[r];
-      const double cn = MJIn * sD[n + NQ * id];
-#pragma unroll
-      for (int s = 0; s < Ns; ++s) {
-        dl[s] -= ci * F[s];
-        dl[s] += F[s] * lgn * cn;
-      }
+    for (int s = 0; s < Ns; ++s) {
+      acc[s] = r == 0 && assign ? dl[s] : acc[s] + dl[s];
+      asm("" : "+v"(acc[s]));  // summed here: the compiler would keep every direction's dl until the end
     }
-#pragma unroll
-    for (int s = 0; s < Ns; ++s) acc[s] = r == 0 && assign ? dl[s] : acc[s] + dl[s];
   });
   for_dirs<0, D>([&](auto R) {
     constexpr int r = decltype(R)::value;
-    const int ir = idx[r];
-    if (ir != 0 && ir != NQ - 1) return;
-    const bool hi = ir != 0;
-    const int nb = hi ? b.nb[2 * r + 1] : b.nb[2 * r];
-    constexpr int span = (NQ - 1) * line_stride<NQ, r>();
-    // a boundary node reads its own state as the neighbour's and replaces it by the boundary state
-    const uint32_t idp = 8 * (nb >= 0 ? (uint32_t)nb * Np + ijk + (hi ? -span : span) : e * Np + ijk);
-    double qp[Ns], ap[NA], nf[Ns];
+    const bool hi = idx[r] != 0;
+    if (hi && idx[r] != NQ - 1) return;
+    const int nb = rec->nb[2 * r + (hi ? 1 : 0)];
+    const uint32_t idp = across<NQ, D>(r, hi, nb, e, ijk);
+    double qp[Ns], ap[NA], sf[Ns];
 #pragma unroll
     for (int s = 0; s < Ns; ++s) qp[s] = ldo(p, q, s, idp);
     box_aux<L>(p, idp, ap);
-    const double sg = hi ? 1.0 : -1.0;
-    if (nb < 0) {
-      double n[D];
+    fd_box_face<L, SF, r>(p, nb, hi ? 1.0 : -1.0, q1, a1, qp, ap, face_weight<D>(sw, idx, r) * rec->fJ[r], MJIn, sf);
 #pragma unroll
-      for (int d = 0; d < D; ++d) n[d] = d == r ? sg : 0.0;
-      boundarystate<L>(p.c, n, q1, -nb, qp);
-#pragma unroll
-      for (int s = 0; s < NA; ++s) ap[s] = a1[s];
-    }
-    axis_ref_flux<L, SF, r>(p.c, sg, q1, a1, qp, ap, nf);
-    double wf = 1.0;
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-      if (d != r) wf = wf * sw[idx[d]];
-    const double fMJ = wf * b.fJ[r];
-#pragma unroll
-    for (int s = 0; s < Ns; ++s) acc[s] -= fMJ * nf[s] * MJIn;
+    for (int s = 0; s < Ns; ++s) acc[s] -= sf[s];
   });
   box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+}
+
+// One thread per node and direction: the waves of group r (blockDim / D threads) form direction r's volume
+// sum and face, and group 0 adds them up in the order above.  The same numbers; a node's chain of
+// pairs, which is all the time a small mesh takes, is D times shorter.
+template <class L, int NQ, int SF>
+ATM_DEV void fd_box_dirs_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
+                              double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
+                              int epw) {
+  using PF = BoxPairEC<L>;
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D), NP = PF::NP;
+  constexpr int stride = (NP + 1 + 2 * (D - 1) * Ns) * Np;
+  double* sD = lds;
+  double* sw = lds + NQ * NQ;
+  const int group = blockDim.x / D;
+  const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / group);  // whole waves
+  const int tid = threadIdx.x - r * group;
+  const int el = tid / Np;
+  const int ijk = tid - el * Np;
+  const uint32_t le = (uint32_t)blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < (uint32_t)p.K;
+  const uint32_t e = (p.sched && active) ? (uint32_t)p.sched[le] : le;
+  double* sP = lds + NQ * NQ + NQ + el * stride;  // [k][node], MJ, then [r - 1][volume, face][s][node]
+  double* sx = sP + (NP + 1) * Np;
+  for (int t = threadIdx.x; t < NQ * NQ; t += blockDim.x) sD[t] = p.D[t];
+  for (int t = threadIdx.x; t < NQ; t += blockDim.x) sw[t] = p.bw[t];
+  double q1[Ns], a1[NA], P1[NP], qp[Ns], ap[NA], dq0[Ns];
+  const uint32_t e0 = active ? e : 0;  // a lane past the last element reads element 0 and discards it
+  const uint32_t node = 8 * (e0 * Np + ijk);
+  int idx[3];
+  node_index<D>(ijk, NQ, idx);
+  const BoxElem<D>* rec = box_elem<D>(p, e0);
+  const int ir = r == 0 ? idx[0] : (r == 1 ? idx[1] : idx[2]);
+  const bool hi = ir != 0, face = ir == 0 || ir == NQ - 1;
+  const int nb = rec->nb[2 * r + (hi ? 1 : 0)];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
+  box_aux<L>(p, node, a1);
+  const double MJn = p.bw[NQ + ijk] * rec->J, g = rec->g[r], fJ = rec->fJ[r];
+  // a node inside the element reads itself
+  const uint32_t idp = face ? across<NQ, D>(r, hi, nb, e0, ijk) : node;
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) qp[s] = ldo(p, q, s, idp);
+  box_aux<L>(p, idp, ap);
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) dq0[s] = assign || r > 0 ? 0.0 : ldo(p, dq, s, node);
+  if (r == 0) {
+    PF::prim(p.c, q1, a1, P1);
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) sP[k * Np + ijk] = P1[k];
+      sP[NP * Np + ijk] = MJn;
+    }
+  }
+  __syncthreads();
+  const double MJIn = fast_rcp(MJn);
+  double dl[Ns], sf[Ns];
+  if (active) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) P1[k] = sP[k * Np + ijk];
+    const double fMJ = face_weight<D>(sw, idx, r) * fJ, sg = hi ? 1.0 : -1.0;
+    for_dirs<0, D>([&](auto R) {
+      constexpr int rc = decltype(R)::value;
+      if (r != rc) return;
+      fd_box_dir<L, NQ, rc>(p, sD, sP, ijk, ir, g, MJn, MJIn, q1, a1, P1, dl);
+      if (face) fd_box_face<L, SF, rc>(p, nb, sg, q1, a1, qp, ap, fMJ, MJIn, sf);
+    });
+    if (r > 0) {
+      double* x = sx + (r - 1) * (2 * Ns * Np) + ijk;
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) x[s * Np] = dl[s];
+      if (face) {
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) x[(Ns + s) * Np] = sf[s];
+      }
+    }
+  }
+  __syncthreads();
+  if (!active || r > 0) return;
+  double acc[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) {
+    acc[s] = assign ? dl[s] : alpha * dq0[s] + dl[s];
+#pragma unroll
+    for (int d = 1; d < D; ++d) acc[s] = acc[s] + sx[((d - 1) * 2 * Ns + s) * Np + ijk];
+    if (face) acc[s] -= sf[s];
+#pragma unroll
+    for (int d = 1; d < D; ++d)
+      if (idx[d] == 0 || idx[d] == NQ - 1) acc[s] -= sx[((d - 1) * 2 * Ns + Ns + s) * Np + ijk];
+  }
+  box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+}
+
+// Largest workgroup of the form with a thread per node and direction: the 2-D kernels' (every shape fits).
+// Per stage, one thread per node against one per node and direction: vortex 8^2 N = 4 12.2 -> 8.2 us,
+// 32^2 N = 3 8.8 -> 6.8, 30^2 N = 7 14.1 -> 12.6, 64^2 N = 4 13.5 -> 13.5, 45^2 N = 6 16.9 -> 16.4.  In 3-D its
+// six-wave workgroups of 168 registers leave too few of them resident: bubble 12^3 N = 4 38 -> 57 us, 14^3
+// N = 3 26.4 -> 30.4.
+template <class L>
+constexpr int fd_box_dirs_threads() {
+  return L::D == 2 ? 1024 : 0;
+}
+
+template <class L, int NQ>
+constexpr size_t fd_box_elem_bytes() {
+  constexpr int planes = BoxPairEC<L>::NP + 1 + (fd_box_dirs_threads<L>() > 0 ? 2 * (L::D - 1) * L::Ns : 0);
+  return sizeof(double) * planes * ipow(NQ, L::D);
+}
+
+template <class L, int NQ, int SF>
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, fd_box_dirs_threads<L>())))
+fd_box_dirs_kernel(const DevDG p, const double* __restrict__ q, double* __restrict__ dq, double alpha, int assign,
+                   double* __restrict__ qout, double bdt, int epw) {
+  extern __shared__ double lds[];
+  fd_box_dirs_body<L, NQ, SF>(p, lds, xcd_block(), q, dq, alpha, assign, qout, bdt, epw);
+}
+
+template <class L, int NQ, int SF>
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, fd_box_dirs_threads<L>())))
+fd_box_dirs_kernel_batch(const BatchEntry* __restrict__ tab, int n, int parity, double alpha, int assign, double b,
+                         int epw) {
+  extern __shared__ double lds[];
+  const int64_t lb = xcd_block();
+  const int i = batch_find(tab, n, lb);
+  const DevDG p = tab[i].p;
+  fd_box_dirs_body<L, NQ, SF>(p, lds, lb - tab[i].block_start, tab[i].buf[parity], tab[i].dq, alpha, assign,
+                              tab[i].buf[1 - parity], b * tab[i].dt, epw);
 }
 
 ATM_KERNEL_PAIR(fd_box_kernel, fd_box_body, class L ATM_COMMA int NQ ATM_COMMA int SF, L ATM_COMMA NQ ATM_COMMA SF)
@@ -259,6 +426,12 @@ hipError_t launch_fd_box(const DevDG& p, hipStream_t st, const double* q, double
   if (p.epw < 1 || threads > 512) return hipErrorInvalidConfiguration;
   const int blocks = (p.K + p.epw - 1) / p.epw;
   if (blocks == 0) return hipSuccess;
+  if constexpr (fd_box_dirs_threads<L>() > 0)
+    if (L::D * threads <= fd_box_dirs_threads<L>()) {
+      hipLaunchKernelGGL((fd_box_dirs_kernel<L, NQ, SF>), dim3(blocks), dim3(L::D * threads), p.lds, st, p, q, dq,
+                         alpha, assign, qout, bdt, p.epw);
+      return hipGetLastError();
+    }
   hipLaunchKernelGGL((fd_box_kernel<L, NQ, SF>), dim3(blocks), dim3(threads), p.lds, st, p, q, dq, alpha, assign, qout,
                      bdt, p.epw);
   return hipGetLastError();
@@ -267,6 +440,12 @@ hipError_t launch_fd_box(const DevDG& p, hipStream_t st, const double* q, double
 template <class L, int NQ, int SF>
 hipError_t launch_fd_box_batch(const BatchEntry* tab, int n, int64_t blocks, int threads, size_t lds, int epw,
                                hipStream_t st, int parity, double alpha, int assign, double b) {
+  if constexpr (fd_box_dirs_threads<L>() > 0)
+    if (L::D * threads <= fd_box_dirs_threads<L>()) {
+      hipLaunchKernelGGL((fd_box_dirs_kernel_batch<L, NQ, SF>), dim3(blocks), dim3(L::D * threads), lds, st, tab, n,
+                         parity, alpha, assign, b, epw);
+      return hipGetLastError();
+    }
   hipLaunchKernelGGL((fd_box_kernel_batch<L, NQ, SF>), dim3(blocks), dim3(threads), lds, st, tab, n, parity, alpha,
                      assign, b, epw);
   return hipGetLastError();
@@ -275,8 +454,9 @@ hipError_t launch_fd_box_batch(const BatchEntry* tab, int n, int64_t blocks, int
 template <class L, int NQ, int SF>
 Resolved make_fd_box() {
   constexpr int Np = ipow(NQ, L::D);
-  return make_resolved(launch_fd_box<L, NQ, SF>, launch_fd_box_batch<L, NQ, SF>, L::Ns, elements_per_workgroup(Np),
-                       sizeof(double) * (NQ * NQ + NQ), sizeof(double) * (BoxPairEC<L>::NP + 1) * Np);
+  // one wave of small elements by default, as the FAST kernels
+  return make_resolved(launch_fd_box<L, NQ, SF>, launch_fd_box_batch<L, NQ, SF>, L::Ns, Np >= 64 ? 1 : 64 / Np,
+                       sizeof(double) * (NQ * NQ + NQ), fd_box_elem_bytes<L, NQ>());
 }
 
 template <class L, int SF>

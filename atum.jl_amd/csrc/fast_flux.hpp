@@ -41,12 +41,20 @@ __device__ __forceinline__ double fast_sqrt(double x) {
   return fma(fma(-g, g, x), h, g);
 }
 
-// a/x from ix = fast_rcp(x): the quotient with one residual correction, which rounds as an IEEE
-// division does
+// a/x from an approximate 1/x (fast_rcp, or rcp_div's 47 bits): the quotient with one residual
+// correction, which rounds as an IEEE division does
 __device__ __forceinline__ double fast_div(double a, double x, double ix) {
 #pragma clang fp contract(fast)
   const double q = a * ix;
   return fma(fma(-x, q, a), ix, q);
+}
+
+// 1/x to 47 bits, one Newton step on the hardware reciprocal: enough for fast_div, whose correction
+// squares the error
+__device__ __forceinline__ double rcp_div(double x) {
+#pragma clang fp contract(fast)
+  const double r = __builtin_amdgcn_rcp(x);
+  return fma(r, fma(-x, r, 1.0), r);
 }
 
 template <class L, int SF>

@@ -107,17 +107,33 @@ ATM_DEV double lm_log_far(double z) {
   return z == 0 ? -HUGE_VAL : (z > 0 ? z : __builtin_nan(""));
 }
 
-// logavg(a, b) of the reference, ib = fast_rcp(b)
-ATM_DEV double lm_logavg(double a, double b, double ib) {
+// logavg(a0, b0) and logavg(a1, b1) of the reference.  Reciprocals are taken in pairs, of the
+// product of the two means' divisors (the hardware's takes four times an FMA): good to 46 bits, which
+// fast_div corrects.
+ATM_DEV void lm_logavg2(double a0, double b0, double a1, double b1, double* m0, double* m1) {
 #pragma clang fp contract(off)
-  const double z = fast_div(a, b, ib);
-  const double s = z + 1, is = fast_rcp(s), f = fast_div(z - 1, s, is), u = f * f, t = 2 * f;
-  double l;
-  if (u < LM_NEAR) l = t + lm_rest(z, s, is, f, u);
-  else l = lm_log_far(z);
-  // below eps the reference's series in u is 1 after rounding
-  const double F = u < 2.220446049250313e-16 ? 1.0 : fast_div(l, t, fast_rcp(t));
-  return fast_div(a + b, 2 * F, fast_rcp(2 * F));
+  constexpr double EPS = 2.220446049250313e-16;
+  const double ib = rcp_div(b0 * b1);
+  const double z0 = fast_div(a0, b0, b1 * ib), z1 = fast_div(a1, b1, b0 * ib);
+  const double s0 = z0 + 1, s1 = z1 + 1, is = rcp_div(s0 * s1), is0 = s1 * is, is1 = s0 * is;
+  const double f0 = fast_div(z0 - 1, s0, is0), f1 = fast_div(z1 - 1, s1, is1);
+  const double u0 = f0 * f0, u1 = f1 * f1;
+  double l0, l1;
+  if (u0 < LM_NEAR && u1 < LM_NEAR) {
+    l0 = 2 * f0 + lm_rest(z0, s0, is0, f0, u0);
+    l1 = 2 * f1 + lm_rest(z1, s1, is1, f1, u1);
+  } else {
+    l0 = lm_log_far(z0);
+    l1 = lm_log_far(z1);
+  }
+  // below eps the reference's series in u is 1 after rounding: l/t with both 1
+  const bool eq0 = u0 < EPS, eq1 = u1 < EPS;
+  const double t0 = eq0 ? 1.0 : 2 * f0, t1 = eq1 ? 1.0 : 2 * f1;
+  const double it = rcp_div(t0 * t1);
+  const double F0 = 2 * fast_div(eq0 ? 1.0 : l0, t0, t1 * it), F1 = 2 * fast_div(eq1 ? 1.0 : l1, t1, t0 * it);
+  const double iF = rcp_div(F0 * F1);
+  *m0 = fast_div(a0 + b0, F0, F1 * iF);
+  *m1 = fast_div(a1 + b1, F1, F0 * iF);
 }
 
 }  // namespace atm
