@@ -187,10 +187,9 @@ ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, uint32_t e
 // Bound by memory traffic.  Against the general kernels, per fused stage: 2-D shallow water, 256^2
 // elements, N = 3: 42.1 -> 28.4 us (134 MB of states: 4.7 TB/s); 3-D Euler, 20^3, N = 4, which had run
 // the runtime-degree kernel: 93.0 -> 49.4 us; 2-D advection, 80^2, N = 4: 6.6 -> 4.7 us.
-template <class L, int NQ, int SF, int MASK>
-ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
-                           double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
-                           int epw) {
+// EP: what a node's tendency goes into; load() is called with the node's other loads, store() last.
+template <class L, int NQ, int SF, int MASK, class EP>
+ATM_DEV void weak_box_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
   constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D);
   double* sD = lds;
   double* sw = lds + NQ * NQ;
@@ -215,13 +214,7 @@ ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
   box_aux<L>(p, node, a1);
   const double wp = p.bw[NQ + ijk];
-  double dq0[Ns];
-#pragma unroll
-  for (int s = 0; s < Ns; ++s) dq0[s] = 0.0;
-  if (!assign) {  // uniform over the launch
-#pragma unroll
-    for (int s = 0; s < Ns; ++s) dq0[s] = ldo(p, dq, s, node);
-  }
+  ep.load(p, node);
   const double MJn = wp * b.J;
   if (active) {
     double F[D][Ns];
@@ -263,9 +256,93 @@ ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   }
   double acc[Ns];
 #pragma unroll
-  for (int s = 0; s < Ns; ++s) acc[s] = assign ? dl[s] : alpha * dq0[s] + dl[s];
+  for (int s = 0; s < Ns; ++s) acc[s] = ep.start(s, dl[s]);
   box_surface_node<L, SF, NQ, MASK>(p, b, e, ijk, idx, q, q1, a1, MJIn, sw, acc);
-  box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+  ep.store(p, node, q1, acc);
+}
+
+// dq = (assign ? 0 : alpha dq) + L(q) and, with qout, the stage's new state
+template <class L>
+struct StageEnd {
+  double* dq;
+  double alpha;
+  int assign;
+  double* qout;
+  double bdt;
+  double dq0[L::Ns];
+  ATM_DEV StageEnd(double* dq, double alpha, int assign, double* qout, double bdt)
+      : dq(dq), alpha(alpha), assign(assign), qout(qout), bdt(bdt) {}
+  ATM_DEV void load(const DevDG& p, uint32_t node) {
+#pragma unroll
+    for (int s = 0; s < L::Ns; ++s) dq0[s] = 0.0;
+    if (!assign) {  // uniform over the launch
+#pragma unroll
+      for (int s = 0; s < L::Ns; ++s) dq0[s] = ldo(p, dq, s, node);
+    }
+  }
+  ATM_DEV double start(int s, double dl) const { return assign ? dl : alpha * dq0[s] + dl; }
+  ATM_DEV void store(const DevDG& p, uint32_t node, const double* q1, const double* acc) const {
+    box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+  }
+};
+
+template <class L, int NQ, int SF, int MASK>
+ATM_DEV void weak_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
+                           double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
+                           int epw) {
+  StageEnd<L> ep(dq, alpha, assign, qout, bdt);
+  weak_box_node<L, NQ, SF, MASK>(p, lds, blk, q, ep, epw);
+}
+
+// The implicit tendency of an ARK stage, added where it is formed to the sums that the explicit and implicit
+// tendencies of the stage go into (ArkSums) instead of being stored and read again by a pass for each
+// sum; the same operations in the same order as those passes.
+template <class L>
+struct ArkEnd {
+  const ArkSums& a;
+  double ex[L::Ns], in[3][L::Ns];
+  ATM_DEV explicit ArkEnd(const ArkSums& a) : a(a) {}
+  ATM_DEV void load(const DevDG& p, uint32_t node) {
+#pragma unroll
+    for (int s = 0; s < L::Ns; ++s) ex[s] = a.ex ? ldo(p, a.ex, s, node) : 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (j < a.n && a.in[j]) {
+#pragma unroll
+        for (int s = 0; s < L::Ns; ++s) in[j][s] = ldo(p, a.in[j], s, node);
+      }
+  }
+  ATM_DEV double start(int, double dl) const { return dl; }
+  ATM_DEV void store(const DevDG& p, uint32_t node, const double* q1, const double* im) const {
+#pragma unroll
+    for (int s = 0; s < L::Ns; ++s) {
+      const double e = a.unsplit ? ex[s] - im[s] : ex[s];
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (j < a.n) {
+          const double v = a.in[j] ? in[j][s] : q1[s];
+          sto(p, a.out[j], s, node, v + a.dt * (a.ea[j] * e + a.ia[j] * im[s]));
+        }
+    }
+  }
+};
+
+template <class L, int NQ, int SF, int MASK>
+__global__ void __launch_bounds__(512)
+    weak_box_ark_kernel(const DevDG p, const double* __restrict__ q, const ArkSums a, int epw) {
+  extern __shared__ double lds[];
+  ArkEnd<L> ep(a);
+  weak_box_node<L, NQ, SF, MASK>(p, lds, xcd_block(), q, ep, epw);
+}
+
+template <class L, int NQ, int SF, int MASK>
+hipError_t launch_weak_box_ark(const DevDG& p, hipStream_t st, const double* q, const ArkSums& a) {
+  const int threads = ((p.epw * p.Np + 63) / 64) * 64;
+  if (p.epw < 1 || threads > 512) return hipErrorInvalidConfiguration;
+  const int blocks = (p.K + p.epw - 1) / p.epw;
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL((weak_box_ark_kernel<L, NQ, SF, MASK>), dim3(blocks), dim3(threads), p.lds, st, p, q, a, p.epw);
+  return hipGetLastError();
 }
 
 ATM_KERNEL_PAIR(weak_box_kernel, weak_box_body, class L ATM_COMMA int NQ ATM_COMMA int SF ATM_COMMA int MASK,
@@ -327,9 +404,12 @@ hipError_t launch_weak_box_batch(const BatchEntry* tab, int n, int64_t blocks, i
 template <class L, int NQ, int SF, int MASK>
 Resolved make_weak_box() {
   constexpr int Np = ipow(NQ, L::D);
-  return make_resolved(launch_weak_box<L, NQ, SF, MASK>, launch_weak_box_batch<L, NQ, SF, MASK>, L::Ns,
-                       elements_per_workgroup(Np), sizeof(double) * (NQ * NQ + NQ),
-                       sizeof(double) * __builtin_popcount(MASK) * L::Ns * Np);
+  Resolved r = make_resolved(launch_weak_box<L, NQ, SF, MASK>, launch_weak_box_batch<L, NQ, SF, MASK>, L::Ns,
+                             elements_per_workgroup(Np), sizeof(double) * (NQ * NQ + NQ),
+                             sizeof(double) * __builtin_popcount(MASK) * L::Ns * Np);
+  // operators of the last direction only are the implicit halves of IMEX pairs
+  if constexpr (L::D > 1 && MASK == 1 << (L::D - 1)) r.afn = launch_weak_box_ark<L, NQ, SF, MASK>;
+  return r;
 }
 
 template <class L, int SF, int MASK>

@@ -612,6 +612,18 @@ size_t lds_elem_bytes(int form, int vflux, int Np) {
   return sizeof(double) * (size_t)(np + D) * Np;
 }
 
+// Sums of an ARK23 step that take a stage's explicit (ex; null: zero) and implicit tendency:
+// out_j = in_j + dt (ea_j ex + ia_j im), in_j the stage's own state where null; out_j may be in_j.
+// unsplit: ex is the full tendency, its explicit part ex - im.
+struct ArkSums {
+  const double* ex;
+  const double* in[3];
+  double* out[3];
+  double ea[3], ia[3], dt;
+  int n, unsplit;
+};
+typedef hipError_t (*ArkFn)(const DevDG& p, hipStream_t st, const double* q, const ArkSums& a);
+
 // A kernel family for an operator: launchers, the default elements per
 // workgroup and the LDS bytes of a workgroup, lds_fixed + epw * lds_elem.
 struct Resolved {
@@ -625,6 +637,7 @@ struct Resolved {
   // batched launcher shared by the members of one family of different Nq (one
   // launch per stage for all of them), or null
   BatchLaunchFn mbfn = nullptr;
+  ArkFn afn = nullptr;  // the tendency added to an ARK step's sums, or null
 };
 
 inline Resolved make_resolved(LaunchFn fn, BatchLaunchFn bfn, int ns, int epw, size_t fixed, size_t elem,

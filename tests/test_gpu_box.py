@@ -138,3 +138,32 @@ def test_fast_box_kernels_against_the_general_ones(law, dim, Kd, kw, sflux, N):
     assert device_bytes(box) > device_bytes(general)
     a, b = tendencies(box, general, q0)
     assert np.abs(a - b).max() <= 2e-12 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("explicit", [True, False])
+@pytest.mark.parametrize("split,paper", [(False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("law,dim,N", [("advection", 2, 4), ("euler_gravity", 2, 3), ("euler_gravity", 3, 3)])
+def test_ark_step_with_sums_in_the_implicit_kernel(law, dim, N, split, paper, explicit):
+    """One ARK23 step whose implicit operator is on box elements (its kernel adds the stages' tendencies up)
+    against the general operators (a pass for each sum): the same operations in the same order, so equal in
+    the columns that the last node's other MJI cannot reach in three tendencies."""
+    import atum_hip as A
+    K = (11, 4) if dim == 2 else (11, 2, 4)
+    lin_law = law if law == "advection" else "linear_euler_gravity"
+    kw = dict(bc="zero_inflow" if law == "advection" else "reflect", periodic=(True,) * (dim - 1) + (False,),
+              ordering="stacked", seed=5)
+    lb, lg, q0 = pair(lin_law, dim, N, K, directions=(dim,), **kw)
+    eb, eg, q0 = pair(law, dim, N, K, **kw)
+    out = []
+    for lin, ex in ((lb, eb), (lg, eg)):
+        q = lin.fieldarray(q0)
+        A.ARK23(ex if explicit else None, lin, q, 1e-3, split_rhs=split, paperversion=paper).run(q, 1)
+        lin.ctx.sync()
+        out.append(q.numpy().reshape(q0.shape[0], lin.grid.K, -1))
+    # stacked elements: the first dimension's index of element e is (e // K[-1]) % K[0]
+    x = (np.arange(lb.grid.K) // K[-1]) % K[0]
+    far = (x >= 3) & (x <= 6)
+    assert np.isfinite(out[0]).all()
+    # (unsplit without an explicit operator the explicit part is minus the implicit one: nothing moves)
+    assert (np.abs(out[0] - q0.reshape(out[0].shape)).max() > 0) == (explicit or split)
+    np.testing.assert_array_equal(out[0][:, far], out[1][:, far])
