@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "dg_kernels.hpp"
+#include "fast_flux.hpp"
 
 namespace atm {
 
@@ -95,56 +96,86 @@ ATM_DEV void for_dirs(F&& f) {
   }
 }
 
-// Wave speed with the unit normal of direction R (the laws' wavespeed with the other
-// components of the normal zero)
-template <class L, int R>
-ATM_DEV double axis_wavespeed(const LawConst& c, const double* q, const double* a) {
-  constexpr int D = L::D;
-  if constexpr (L::LAW == ATM_LAW_ADVECTION) {
-    return fabs(c.u[R]);
-  } else if constexpr (L::LAW == ATM_LAW_LINEAR_EULER_GRAVITY) {
-    return L::wavespeed(c, nullptr, q, a);
-  } else if constexpr (L::LAW == ATM_LAW_SHALLOW_WATER) {
-    return fabs(q[1 + R] / q[0]) + sqrt(c.grav * q[0]);
-  } else {
-    double p;
-    if constexpr (L::LAW == ATM_LAW_EULER_GRAVITY) p = L::pressure(c, q[0], q + 1, q[D + 1], a[0]);
-    else p = L::pressure(c, q[0], q + 1, q[D + 1]);
-    return fabs(q[1 + R] / q[0]) + sqrt(c.gamma * p / q[0]);
-  }
-}
+// What the weak form takes of a state: row<R>() is the law's flux in direction R, speed<R>() its wave speed with
+// the unit normal of direction R.  A node forms its own once, for its flux and all its faces.  The quotients by
+// one density share a reciprocal and are corrected (fast_div), so they and the roots (fast_sqrt) are the law's.
+template <class L, int LAW = L::LAW>
+struct WeakSide;
 
-// surfaceflux<L, SF> with the normal sg * e_R, sg = +-1: the products with the normal's zeros
-// and ones are left out, so the result is the same value (up to the sign of a zero)
-template <class L, int SF, int R>
-ATM_DEV void axis_surfaceflux(const LawConst& c, double sg, const double* qm, const double* am, const double* qp,
-                              const double* ap, double* nf) {
-  constexpr int D = L::D, Ns = L::Ns;
-  if constexpr (SF == ATM_FLUX_ROE || SF == ATM_FLUX_MATRIX) {
-    double n[D];
+template <class L>
+struct WeakSide<L, ATM_LAW_ADVECTION> {
+  ATM_DEV WeakSide(const LawConst&, const double*, const double*) {}
+  template <int R>
+  ATM_DEV void row(const LawConst& c, const double* q, double* f) const { f[0] = c.u[R] * q[0]; }
+  template <int R>
+  ATM_DEV double speed(const LawConst& c) const { return fabs(c.u[R]); }
+};
+
+// root of a squared sound speed: fast_sqrt, and 0 for 0
+ATM_DEV double speed_root(double x) { return x == 0 ? x : fast_sqrt(x); }
+
+template <class L>
+struct WeakSide<L, ATM_LAW_LINEAR_EULER_GRAVITY> {
+  static constexpr int D = L::D;
+  double p, h, cs;
+  ATM_DEV WeakSide(const LawConst& c, const double* q, const double* a) {
+    const double phi = a[0], rho = a[D + 1], ref_p = a[D + 2], gm1 = c.gamma - 1;
+    const double ir = rcp_div(rho);
+    p = gm1 * (q[D + 1] - q[0] * phi);
+    const double ref_rhoe = fast_div(ref_p, gm1, rcp_div(gm1)) + rho * phi;
+    h = fast_div(ref_rhoe + ref_p, rho, ir);
+    cs = speed_root(fast_div(c.gamma * ref_p, rho, ir));
+  }
+  template <int R>
+  ATM_DEV void row(const LawConst&, const double* q, double* f) const {
+    f[0] = q[1 + R];
 #pragma unroll
-    for (int d = 0; d < D; ++d) n[d] = d == R ? sg : 0.0;
-    L::template special_surface<SF>(c, n, qm, am, qp, ap, nf);
-  } else {
-    double F[D][Ns];
-    constexpr int TP = (SF == ATM_FLUX_RUSANOV) ? ATM_FLUX_CENTRAL : SF;
-    L::template twopoint<TP>(c, qm, am, qp, ap, F);
+    for (int d = 0; d < D; ++d) f[1 + d] = d == R ? p : 0.0;
+    f[D + 1] = h * q[1 + R];
+  }
+  template <int R>
+  ATM_DEV double speed(const LawConst&) const { return cs; }
+};
+
+// the laws with velocities: Euler, with or without gravity, and shallow water
+template <class L, int LAW>
+struct WeakSide {
+  static constexpr int D = L::D;
+  static constexpr bool SW = LAW == ATM_LAW_SHALLOW_WATER, GRAV = LAW == ATM_LAW_EULER_GRAVITY;
+  double u[D], p, dp, cs;  // velocity, pressure, pressure in the momentum flux, sound speed
+  ATM_DEV WeakSide(const LawConst& c, const double* q, const double* a) {
+    const double rho = q[0], ir = rcp_div(rho);
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) nf[s] = sg * F[R][s];
-    if constexpr (SF == ATM_FLUX_RUSANOV) {
-      const double ws = fmax(axis_wavespeed<L, R>(c, qm, am), axis_wavespeed<L, R>(c, qp, ap));
-#pragma unroll
-      for (int s = 0; s < Ns; ++s) nf[s] = nf[s] - ws * (qp[s] - qm[s]) / 2;
+    for (int d = 0; d < D; ++d) u[d] = fast_div(q[1 + d], rho, ir);
+    if constexpr (SW) {
+      p = dp = c.grav * (rho * rho) / 2;
+      cs = speed_root(c.grav * rho);
+    } else {
+      const double k = 0.5 * fast_div(dotv<D>(q + 1, q + 1), rho, ir);
+      p = GRAV ? (c.gamma - 1) * (q[D + 1] - k - rho * a[0]) : (c.gamma - 1) * (q[D + 1] - k);
+      dp = p;
+      if constexpr (GRAV)
+        if (c.pde_level_balance) dp -= a[D + 2];
+      cs = speed_root(fast_div(c.gamma * p, rho, ir));
     }
   }
-}
+  template <int R>
+  ATM_DEV void row(const LawConst&, const double* q, double* f) const {
+    f[0] = q[1 + R];
+#pragma unroll
+    for (int d = 0; d < D; ++d) f[1 + d] = d == R ? q[1 + R] * u[d] + dp : q[1 + R] * u[d];
+    f[D + 1] = SW ? u[R] * q[D + 1] : u[R] * (q[D + 1] + p);
+  }
+  template <int R>
+  ATM_DEV double speed(const LawConst&) const { return fabs(u[R]) + cs; }
+};
 
 // Surface contributions of the faces this node lies on, subtracted from acc (surface_node on
 // box elements).  sw: the LGL weights.
-template <class L, int SF, int NQ, int MASK>
+template <class L, int NQ, int MASK>
 ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, uint32_t e, int ijk, const int idx[3],
-                              const double* q, const double* qn, const double* an, double MJIn, const double* sw,
-                              double* acc) {
+                              const double* q, const double* qn, const double* an, const WeakSide<L>& own, double MJIn,
+                              const double* sw, double* acc) {
   constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D);
   for_dirs<0, D>([&](auto R) {
     constexpr int r = decltype(R)::value;
@@ -169,7 +200,15 @@ ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, uint32_t e
 #pragma unroll
       for (int s = 0; s < NA; ++s) ap[s] = an[s];
     }
-    axis_surfaceflux<L, SF, r>(p.c, sg, qn, an, qp, ap, nf);
+    // Rusanov with the normal sg * e_r: the products with the normal's zeros and ones are left out, so the
+    // result is the same value (up to the sign of a zero)
+    const WeakSide<L> other(p.c, qp, ap);
+    double fn[Ns], fp[Ns];
+    own.template row<r>(p.c, qn, fn);
+    other.template row<r>(p.c, qp, fp);
+    const double ws = fmax(own.template speed<r>(p.c), other.template speed<r>(p.c));
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) nf[s] = sg * ((fn[s] + fp[s]) / 2) - ws * (qp[s] - qn[s]) / 2;
     double wf = 1.0;
 #pragma unroll
     for (int d = 0; d < D; ++d)
@@ -184,9 +223,14 @@ ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, uint32_t e
 // Weak form on box elements: weak_body with the compact geometry, the same operations in the
 // same order.  Only the flux row of a direction enters its sum (the metric is diagonal), and
 // LDS holds only the directions of the operator (the bits of MASK, fixed at compile time).
-// Bound by memory traffic.  Against the general kernels, per fused stage: 2-D shallow water, 256^2
-// elements, N = 3: 42.1 -> 28.4 us (134 MB of states: 4.7 TB/s); 3-D Euler, 20^3, N = 4, which had run
-// the runtime-degree kernel: 93.0 -> 49.4 us; 2-D advection, 80^2, N = 4: 6.6 -> 4.7 us.
+// Bound by vector instructions and memory traffic about equally (3-D Euler, N = 4: 830 instructions a
+// wave, the vector units 70 % busy; they were 1195 when every face formed both sides' law terms with IEEE
+// divisions).  Against the general kernels, per fused stage: 2-D shallow water, 256^2 elements, N = 3:
+// 42.1 -> 25.9 us (134 MB of states: 5.2 TB/s); 3-D Euler, 20^3, N = 4, which had run the runtime-degree
+// kernel: 93.0 -> 39.5 us; 2-D advection, 80^2, N = 4: 6.6 -> 4.6 us.
+// The sum over n stays a loop: unrolled, its LDS reads in flight took 30 registers more, which cost
+// waves: 40 shallow-water meshes of mixed degree 920 -> 846 us, 3-D Euler 9^3, N = 7 248 -> 195 us a pass
+// of 10 stages, shallow water 175^2, N = 7 500 -> 479 us; no size measured was slower by more than 2 %.
 // EP: what a node's tendency goes into; load() is called with the node's other loads, store() last.
 template <class L, int NQ, int SF, int MASK, class EP>
 ATM_DEV void weak_box_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
@@ -216,26 +260,26 @@ ATM_DEV void weak_box_node(const DevDG& p, double* lds, int64_t blk, const doubl
   const double wp = p.bw[NQ + ijk];
   ep.load(p, node);
   const double MJn = wp * b.J;
+  const WeakSide<L> own(p.c, q1, a1);
   if (active) {
-    double F[D][Ns];
-    L::flux(p.c, q1, a1, F);
-    int slot = 0;
+    for_dirs<0, D>([&](auto R) {
+      constexpr int r = decltype(R)::value, slot = __builtin_popcount(MASK & ((1 << r) - 1));
+      if constexpr ((MASK >> r) & 1) {
+        double F[Ns];
+        own.template row<r>(p.c, q1, F);
 #pragma unroll
-    for (int r = 0; r < D; ++r) {
-      if (!((MASK >> r) & 1)) continue;
-#pragma unroll
-      for (int s = 0; s < Ns; ++s) slF[(slot * Ns + s) * Np + ijk] = b.g[r] * F[r][s] * MJn;
-      ++slot;
-    }
+        for (int s = 0; s < Ns; ++s) slF[(slot * Ns + s) * Np + ijk] = b.g[r] * F[s] * MJn;
+      }
+    });
   }
   __syncthreads();
   if (!active) return;
-  const double MJIn = 1 / MJn;
+  const double MJIn = fast_div(1.0, MJn, rcp_div(MJn));
   double dl[Ns];
 #pragma unroll
   for (int s = 0; s < Ns; ++s) dl[s] = -0.0;
   L::sources(p.c, dl, q1, a1, MASK, true);
-#pragma unroll
+#pragma unroll 1
   for (int n = 0; n < NQ; ++n) {
     double Dn[D];
 #pragma unroll
@@ -257,7 +301,7 @@ ATM_DEV void weak_box_node(const DevDG& p, double* lds, int64_t blk, const doubl
   double acc[Ns];
 #pragma unroll
   for (int s = 0; s < Ns; ++s) acc[s] = ep.start(s, dl[s]);
-  box_surface_node<L, SF, NQ, MASK>(p, b, e, ijk, idx, q, q1, a1, MJIn, sw, acc);
+  box_surface_node<L, NQ, MASK>(p, b, e, ijk, idx, q, q1, a1, own, MJIn, sw, acc);
   ep.store(p, node, q1, acc);
 }
 

@@ -91,6 +91,17 @@ def test_weak_box_kernels_equal_the_general_ones(law, dim, Kd, kw, N):
     np.testing.assert_array_equal(a[:, :-1], b[:, :-1])
 
 
+@pytest.mark.parametrize("dim,Kd", [(1, (6,)), (2, (4, 3)), (3, (2, 3, 2))])
+def test_weak_box_kernels_without_pressure(dim, Kd):
+    """A sound speed of zero: the root of the box kernels is that of the general ones there too."""
+    box, general, q0 = pair("euler", dim, 3, Kd, seed=5)
+    rho = 2.0 ** np.random.default_rng(1).integers(-2, 3, q0[0].shape)
+    q0[0], q0[1:-1], q0[-1] = rho, rho, dim * rho / 2  # velocity 1, all energy kinetic
+    a, b = tendencies(box, general, q0)
+    assert np.isfinite(a).all()
+    np.testing.assert_array_equal(a[:, :-1], b[:, :-1])
+
+
 @pytest.mark.parametrize("dim,Kd", [(1, (5,)), (2, (4, 3)), (3, (3, 2, 2))])
 def test_device_built_and_host_built_boxes_agree(dim, Kd):
     import atum_hip as A
