@@ -177,6 +177,7 @@ void dg_use_box(atm_dg* dg, const Resolved& r, const void* rec, const double* ta
   dg->bfn = r.bfn;
   dg->mbfn = r.mbfn;
   dg->afn = r.afn;
+  dg->pfn = r.pfn;
   dg->lds = r.lds;
   dg->epw = r.epw;
   dg->lds_fixed = r.lds_fixed;

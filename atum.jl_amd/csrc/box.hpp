@@ -12,6 +12,7 @@
 // bit for bit in every node and face point, so that both forms of a kernel compute with the
 // same numbers.  Operators with any other element keep the general kernels.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "dg_kernels.hpp"
@@ -325,6 +326,7 @@ struct StageEnd {
     }
   }
   ATM_DEV double start(int s, double dl) const { return assign ? dl : alpha * dq0[s] + dl; }
+  ATM_DEV double start_fused(int s, double dl) const { return assign ? dl : fma(alpha, dq0[s], dl); }
   ATM_DEV void store(const DevDG& p, uint32_t node, const double* q1, const double* acc) const {
     box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
   }
@@ -349,6 +351,9 @@ struct ArkEnd {
   ATM_DEV void load(const DevDG& p, uint32_t node) {
 #pragma unroll
     for (int s = 0; s < L::Ns; ++s) ex[s] = a.ex ? ldo(p, a.ex, s, node) : 0.0;
+    load_sums(p, node);
+  }
+  ATM_DEV void load_sums(const DevDG& p, uint32_t node) {
 #pragma unroll
     for (int j = 0; j < 3; ++j)
       if (j < a.n && a.in[j]) {
@@ -370,6 +375,66 @@ struct ArkEnd {
     }
   }
 };
+
+// An explicit tendency that stays with its node's thread (out: registers)
+template <class L>
+struct KeepEnd {
+  double* out;
+  ATM_DEV void load(const DevDG&, uint32_t) {}
+  ATM_DEV double start(int, double dl) const { return dl; }
+  ATM_DEV double start_fused(int, double dl) const { return dl; }
+  ATM_DEV void store(const DevDG&, uint32_t, const double*, const double* acc) const {
+#pragma unroll
+    for (int s = 0; s < L::Ns; ++s) out[s] = acc[s];
+  }
+};
+
+// ArkEnd with the explicit tendency given
+template <class L>
+struct ArkKeptEnd : ArkEnd<L> {
+  ATM_DEV ArkKeptEnd(const ArkSums& a, const double* kept) : ArkEnd<L>(a) {
+#pragma unroll
+    for (int s = 0; s < L::Ns; ++s) this->ex[s] = kept[s];
+  }
+  ATM_DEV void load(const DevDG& p, uint32_t node) { this->load_sums(p, node); }
+};
+
+// The explicit and the implicit tendency of an ARK stage in one launch, for an Euler law with gravity and its
+// linearized law in the vertical on the same elements: BODY forms the explicit tendency (an element kernel's
+// body, all threads come back from it), which its node's thread keeps, and the weak vertical form follows,
+// its state still in the caches.  The same numbers as from two launches, which write and read the
+// explicit tendency and read the state again: 32x32x10 elements, N = 3, 29 + 26 us -> 46 us a stage (FAST).
+template <class L>
+using LinearOf = LinearEulerGravity<L::D>;
+
+template <class L, int NQ, class BODY>
+ATM_DEV void box_ark_pair(const DevDG& p, const DevDG& pl, double* lds, const double* __restrict__ q, const ArkSums& a,
+                          int epw) {
+  using LL = LinearOf<L>;
+  const int64_t blk = xcd_block();
+  double ex[L::Ns];
+#pragma unroll
+  for (int s = 0; s < L::Ns; ++s) ex[s] = 0.0;
+  KeepEnd<L> keep{ex};
+  BODY::run(p, lds, blk, q, keep, epw);
+  __syncthreads();  // the explicit form's LDS is free
+  ArkKeptEnd<LL> ep(a, ex);
+  weak_box_node<LL, NQ, ATM_FLUX_RUSANOV, 1 << (L::D - 1)>(pl, lds, blk, q, ep, epw);
+}
+
+template <class L, int NQ, class KERNEL>
+hipError_t launch_box_ark_pair(KERNEL kernel, int max_threads, const DevDG& p, const DevDG& pl, hipStream_t st,
+                               const double* q, const ArkSums& a) {
+  constexpr int Np = ipow(NQ, L::D);
+  const int threads = ((p.epw * Np + 63) / 64) * 64;
+  if (p.epw < 1 || threads > max_threads) return hipErrorInvalidConfiguration;
+  const int blocks = (p.K + p.epw - 1) / p.epw;
+  if (blocks == 0) return hipSuccess;
+  // the explicit form's LDS holds the implicit one's: the tables and Ns planes of an element
+  const int lds = std::max<int>(p.lds, (int)sizeof(double) * (NQ * NQ + NQ + p.epw * L::Ns * Np));
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), lds, st, p, pl, q, a, p.epw);
+  return hipGetLastError();
+}
 
 template <class L, int NQ, int SF, int MASK>
 __global__ void __launch_bounds__(512)

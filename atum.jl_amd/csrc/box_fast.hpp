@@ -286,10 +286,8 @@ struct BoxFaces {
   }
 };
 
-template <class L, int NQ, int SF>
-ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
-                           double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
-                           int epw) {
+template <class L, int NQ, int SF, class EP>
+ATM_DEV void fast_box_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
 #pragma clang fp contract(fast)
   constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
   using EC = BoxEC<L>;
@@ -417,17 +415,41 @@ ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const doubl
   if (active) bf.run(p, rec, e, ijk, q, sx, sQ, siw[0]);
   __syncthreads();
   if (!active) return;
-  double dq0[Ns];
-#pragma unroll
-  for (int s = 0; s < Ns; ++s) dq0[s] = assign ? 0.0 : ldo(p, dq, s, node);
+  ep.load(p, node);
 #pragma unroll
   for (int s = 0; s < Ns; ++s) q1[s] = sQ[s * Np + ijk];
-  if (!assign) {
 #pragma unroll
-    for (int s = 0; s < Ns; ++s) acc[s] += alpha * dq0[s];
-  }
+  for (int s = 0; s < Ns; ++s) acc[s] = ep.start_fused(s, acc[s]);
   BF::gather(idx, sx, acc);
-  box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+  ep.store(p, node, q1, acc);
+}
+
+template <class L, int NQ, int SF>
+ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
+                           double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
+                           int epw) {
+  StageEnd<L> ep(dq, alpha, assign, qout, bdt);
+  fast_box_node<L, NQ, SF>(p, lds, blk, q, ep, epw);
+}
+
+template <class L, int NQ, int SF>
+struct FastBoxBody {
+  template <class EP>
+  ATM_DEV static void run(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
+    fast_box_node<L, NQ, SF>(p, lds, blk, q, ep, epw);
+  }
+};
+
+template <class L, int NQ, int SF>
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, fast_max_threads<L, NQ, SF>())))
+fast_box_ark_kernel(const DevDG p, const DevDG pl, const double* __restrict__ q, const ArkSums a, int epw) {
+  extern __shared__ double lds[];
+  box_ark_pair<L, NQ, FastBoxBody<L, NQ, SF>>(p, pl, lds, q, a, epw);
+}
+
+template <class L, int NQ, int SF>
+hipError_t launch_fast_box_ark(const DevDG& p, const DevDG& pl, hipStream_t st, const double* q, const ArkSums& a) {
+  return launch_box_ark_pair<L, NQ>(fast_box_ark_kernel<L, NQ, SF>, fast_max_threads<L, NQ, SF>(), p, pl, st, q, a);
 }
 
 template <class L, int NQ, int SF>
@@ -521,6 +543,7 @@ Resolved fast_box_variant() {
                              fast_box_epw<L, NQ, SF>(), sizeof(double) * (NQ * NQ + NQ),
                              sizeof(double) * fast_box_elem_doubles<L, NQ>(), fast_max_threads<L, NQ, SF>());
   if constexpr (NQ >= 4 && NQ <= 8) r.mbfn = launch_fast_box_multi_batch<L, SF>;
+  if constexpr (L::LAW == ATM_LAW_EULER_GRAVITY) r.pfn = launch_fast_box_ark<L, NQ, SF>;
   return r;
 }
 

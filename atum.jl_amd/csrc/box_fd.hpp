@@ -224,10 +224,8 @@ ATM_DEV double face_weight(const double* sw, const int idx[3], int r) {
 }
 
 // One thread per node: the directions one after the other.
-template <class L, int NQ, int SF>
-ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
-                         double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
-                         int epw) {
+template <class L, int NQ, int SF, class EP>
+ATM_DEV void fd_box_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
   using PF = BoxPairEC<L>;
   constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D), NP = PF::NP;
   double* sD = lds;
@@ -261,15 +259,14 @@ ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double*
   if (!active) return;
   const double MJIn = fast_rcp(MJn);
   double acc[Ns];
-#pragma unroll
-  for (int s = 0; s < Ns; ++s) acc[s] = assign ? 0.0 : alpha * ldo(p, dq, s, node);
+  ep.load(p, node);
   for_dirs<0, D>([&](auto R) {
     constexpr int r = decltype(R)::value;
     double dl[Ns];
     fd_box_dir<L, NQ, r>(p, sD, sP, ijk, idx[r], rec->g[r], MJn, MJIn, q1, a1, P1, dl);
 #pragma unroll
     for (int s = 0; s < Ns; ++s) {
-      acc[s] = r == 0 && assign ? dl[s] : acc[s] + dl[s];
+      acc[s] = r == 0 ? ep.start(s, dl[s]) : acc[s] + dl[s];
       asm("" : "+v"(acc[s]));  // summed here: the compiler would keep every direction's dl until the end
     }
   });
@@ -287,7 +284,35 @@ ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double*
 #pragma unroll
     for (int s = 0; s < Ns; ++s) acc[s] -= sf[s];
   });
-  box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
+  ep.store(p, node, q1, acc);
+}
+
+template <class L, int NQ, int SF>
+ATM_DEV void fd_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
+                         double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
+                         int epw) {
+  StageEnd<L> ep(dq, alpha, assign, qout, bdt);
+  fd_box_node<L, NQ, SF>(p, lds, blk, q, ep, epw);
+}
+
+template <class L, int NQ, int SF>
+struct FdBoxBody {
+  template <class EP>
+  ATM_DEV static void run(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
+    fd_box_node<L, NQ, SF>(p, lds, blk, q, ep, epw);
+  }
+};
+
+template <class L, int NQ, int SF>
+__global__ void __launch_bounds__(512)
+    fd_box_ark_kernel(const DevDG p, const DevDG pl, const double* __restrict__ q, const ArkSums a, int epw) {
+  extern __shared__ double lds[];
+  box_ark_pair<L, NQ, FdBoxBody<L, NQ, SF>>(p, pl, lds, q, a, epw);
+}
+
+template <class L, int NQ, int SF>
+hipError_t launch_fd_box_ark(const DevDG& p, const DevDG& pl, hipStream_t st, const double* q, const ArkSums& a) {
+  return launch_box_ark_pair<L, NQ>(fd_box_ark_kernel<L, NQ, SF>, 512, p, pl, st, q, a);
 }
 
 // One thread per node and direction: the waves of group r (blockDim / D threads) form direction r's volume
@@ -455,8 +480,10 @@ template <class L, int NQ, int SF>
 Resolved make_fd_box() {
   constexpr int Np = ipow(NQ, L::D);
   // one wave of small elements by default, as the FAST kernels
-  return make_resolved(launch_fd_box<L, NQ, SF>, launch_fd_box_batch<L, NQ, SF>, L::Ns, Np >= 64 ? 1 : 64 / Np,
-                       sizeof(double) * (NQ * NQ + NQ), fd_box_elem_bytes<L, NQ>());
+  Resolved r = make_resolved(launch_fd_box<L, NQ, SF>, launch_fd_box_batch<L, NQ, SF>, L::Ns, Np >= 64 ? 1 : 64 / Np,
+                             sizeof(double) * (NQ * NQ + NQ), fd_box_elem_bytes<L, NQ>());
+  if constexpr (L::LAW == ATM_LAW_EULER_GRAVITY && L::D == 3) r.pfn = launch_fd_box_ark<L, NQ, SF>;
+  return r;
 }
 
 template <class L, int SF>

@@ -623,6 +623,8 @@ struct ArkSums {
   int n, unsplit;
 };
 typedef hipError_t (*ArkFn)(const DevDG& p, hipStream_t st, const double* q, const ArkSums& a);
+// p, pl: the explicit operator and its linearized vertical one
+typedef hipError_t (*ArkPairFn)(const DevDG& p, const DevDG& pl, hipStream_t st, const double* q, const ArkSums& a);
 
 // A kernel family for an operator: launchers, the default elements per
 // workgroup and the LDS bytes of a workgroup, lds_fixed + epw * lds_elem.
@@ -638,6 +640,7 @@ struct Resolved {
   // launch per stage for all of them), or null
   BatchLaunchFn mbfn = nullptr;
   ArkFn afn = nullptr;  // the tendency added to an ARK step's sums, or null
+  ArkPairFn pfn = nullptr;  // this (explicit) tendency and the implicit one in one launch, or null
 };
 
 inline Resolved make_resolved(LaunchFn fn, BatchLaunchFn bfn, int ns, int epw, size_t fixed, size_t elem,

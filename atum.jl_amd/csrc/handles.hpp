@@ -39,6 +39,7 @@ struct atm_dg {
   int max_threads = 512;               // largest workgroup of the element kernels
   BatchLaunchFn mbfn = nullptr;         // one-launch batched kernel across Nq (or null)
   ArkFn afn = nullptr;                  // ARK form of the element kernel (or null)
+  ArkPairFn pfn = nullptr;              // ARK form with the implicit operator's (or null)
   int32_t* sched = nullptr;             // device copy of the element processing order (or null)
   int law = 0, dim = 0, Nq = 0, Np = 0, Ns = 0;
   int64_t Ntot = 0;

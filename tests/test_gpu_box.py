@@ -178,3 +178,26 @@ def test_ark_step_with_sums_in_the_implicit_kernel(law, dim, N, split, paper, ex
     # (unsplit without an explicit operator the explicit part is minus the implicit one: nothing moves)
     assert (np.abs(out[0] - q0.reshape(out[0].shape)).max() > 0) == (explicit or split)
     np.testing.assert_array_equal(out[0][:, far], out[1][:, far])
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("precision,dim,sflux", [("fast", 2, "roe"), ("fast", 3, "rusanov"), ("fast", 3, "roe"),
+                                                 ("reference", 3, "roe"), ("reference", 3, "rusanov"),
+                                                 ("reference", 2, "roe")])
+def test_ark_stage_in_one_launch(precision, dim, sflux, N):
+    """Both tendencies of a stage in one launch against two launches (an element order set on the explicit
+    operator, the mesh's own, takes them apart): the same numbers."""
+    import atum_hip as A
+    K = (3, 4) if dim == 2 else (3, 2, 4)
+    kw = dict(bc="reflect", periodic=(True,) * (dim - 1) + (False,), ordering="stacked", seed=N)
+    lin, _, q0 = pair("linear_euler_gravity", dim, N, K, directions=(dim,), **kw)
+    ex, _, q0 = pair("euler_gravity", dim, N, K, form="ec", sflux=sflux, precision=precision, **kw)
+    out = []
+    for order in (None, np.arange(lin.grid.K)):
+        ex.set_schedule(order)
+        q = lin.fieldarray(q0)
+        A.ARK23(ex, lin, q, 1e-3, split_rhs=False).run(q, 2)
+        lin.ctx.sync()
+        out.append(q.numpy())
+    assert np.isfinite(out[0]).all() and np.abs(out[0] - q0).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
