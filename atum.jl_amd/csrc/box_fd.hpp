@@ -406,6 +406,157 @@ ATM_DEV void fd_box_dirs_body(const DevDG& p, double* lds, int64_t blk, const do
   box_epilogue<L>(p, node, q1, acc, dq, qout, bdt);
 }
 
+// Workgroups of the form that deals a line's pairs out: twelve waves leave each 168 registers
+constexpr int FD_PAIRS_THREADS = 768;
+
+// The pairs of a line dealt out too: group (r, g) forms direction r's pairs with the partners n = g, g + G, ...
+// and leaves their fluxes in LDS; group (r, 0) then adds them up in the order of fd_box_dir while the last one,
+// (r, G - 1), forms the face, and group (0, 0) puts the directions together.  The same numbers.  A small mesh
+// is bound by one node's chain of pairs (128 waves, bubble 4^3 N = 4, take 14 us a stage, 9 cycles an
+// instruction), which this makes G times shorter.
+template <class L, int NQ>
+struct FdPairs {
+  static constexpr int D = L::D, Ns = L::Ns, Np = ipow(NQ, D), NP = BoxPairEC<L>::NP;
+  static constexpr int NF = D * NQ * Ns;  // flux planes, [r][n][s]
+  // planes: primitives, MJ, fluxes, then [r][volume, face][s]
+  static constexpr int stride = (NP + 1 + NF + 2 * D * Ns) * Np;
+  // groups of partners for workgroups of `threads` per group (1: none)
+  static constexpr int groups(int threads) {
+    const int g = FD_PAIRS_THREADS / (D * threads);
+    return g > NQ ? NQ : g;
+  }
+  static constexpr size_t lds(int epw) { return sizeof(double) * (size_t)(NQ * NQ + NQ + epw * stride); }
+};
+
+template <class L, int NQ, int SF, class EP>
+ATM_DEV void fd_box_pairs_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw,
+                               int group) {
+  using PF = BoxPairEC<L>;
+  using S = FdPairs<L, NQ>;
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = S::Np, NP = S::NP;
+  double* sD = lds;
+  double* sw = lds + NQ * NQ;
+  const int G = blockDim.x / (D * group);
+  const int rg = __builtin_amdgcn_readfirstlane(threadIdx.x / group);  // whole waves
+  const int r = rg / G, gr = rg - r * G;
+  const int tid = threadIdx.x - rg * group;
+  const int el = tid / Np;
+  const int ijk = tid - el * Np;
+  const uint32_t le = (uint32_t)blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < (uint32_t)p.K;
+  const uint32_t e = (p.sched && active) ? (uint32_t)p.sched[le] : le;
+  // a lane past the last element reads element 0 and discards it; its LDS is never written
+  double* sP = lds + NQ * NQ + NQ + (active ? el : 0) * S::stride;
+  double* sF = sP + (NP + 1) * Np;
+  double* sx = sF + S::NF * Np;
+  for (int t = threadIdx.x; t < NQ * NQ; t += blockDim.x) sD[t] = p.D[t];
+  for (int t = threadIdx.x; t < NQ; t += blockDim.x) sw[t] = p.bw[t];
+  double q1[Ns], a1[NA], qp[Ns], ap[NA];
+  const uint32_t e0 = active ? e : 0;
+  const uint32_t node = 8 * (e0 * Np + ijk);
+  int idx[3];
+  node_index<D>(ijk, NQ, idx);
+  const BoxElem<D>* rec = box_elem<D>(p, e0);
+  const int ir = r == 0 ? idx[0] : (r == 1 ? idx[1] : idx[2]);
+  const bool hi = ir != 0, face = (ir == 0 || ir == NQ - 1) && gr == G - 1;
+  const int nb = rec->nb[2 * r + (hi ? 1 : 0)];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
+  box_aux<L>(p, node, a1);
+  const double MJn = p.bw[NQ + ijk] * rec->J, g = rec->g[r], fJ = rec->fJ[r];
+  // a node inside the element, or of a group that takes no face, reads itself
+  const uint32_t idp = face ? across<NQ, D>(r, hi, nb, e0, ijk) : node;
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) qp[s] = ldo(p, q, s, idp);
+  box_aux<L>(p, idp, ap);
+  if (rg == 0) {
+    ep.load(p, node);
+    double P1[NP];
+    PF::prim(p.c, q1, a1, P1);
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < NP; ++k) sP[k * Np + ijk] = P1[k];
+      sP[NP * Np + ijk] = MJn;
+    }
+  }
+  __syncthreads();
+  const double MJIn = fast_rcp(MJn);
+  const double gm1x2 = 2 * (p.c.gamma - 1);
+  if (active) {
+    double P1[NP];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) P1[k] = sP[k * Np + ijk];
+    const double ib2 = fast_rcp(2 * P1[D + 1]);
+    for_dirs<0, D>([&](auto R) {
+      constexpr int rc = decltype(R)::value, st = line_stride<NQ, rc>();
+      if (r != rc) return;
+      const double* line = sP + ijk - ir * st;
+#pragma unroll 1
+      for (int n = gr; n < NQ; n += G) {
+        double P2[NP], F[Ns];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) P2[k] = line[k * Np + n * st];
+        PF::template pair<rc>(gm1x2, P1, ib2, P2, F);
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) sF[((rc * NQ + n) * Ns + s) * Np + ijk] = F[s];
+      }
+    });
+  }
+  __syncthreads();  // fluxes written
+  if (active) {
+    if (gr == 0) {
+      double dl[Ns];
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) dl[s] = -0.0;
+      for_dirs<0, D>([&](auto R) {
+        constexpr int rc = decltype(R)::value;
+        if (r == rc) L::sources(p.c, dl, q1, a1, 1 << rc, false);
+      });
+      const double lgi = MJn * g;
+      const int st = r == 0 ? 1 : (r == 1 ? NQ : NQ * NQ);
+      const double* mj = sP + NP * Np + ijk - ir * st;
+      const double* F = sF + r * NQ * Ns * Np + ijk;
+#pragma unroll 1
+      for (int n = 0; n < NQ; ++n) {
+        const double ci = MJIn * sD[ir + NQ * n] * lgi;
+        const double lgn = mj[n * st] * g;
+        const double cn = MJIn * sD[n + NQ * ir];
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) {
+          const double f = F[(n * Ns + s) * Np];
+          dl[s] -= ci * f;
+          dl[s] += f * lgn * cn;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) sx[(2 * r * Ns + s) * Np + ijk] = dl[s];
+    }
+    if (face) {
+      double sf[Ns];
+      const double fMJ = face_weight<D>(sw, idx, r) * fJ, sg = hi ? 1.0 : -1.0;
+      for_dirs<0, D>([&](auto R) {
+        constexpr int rc = decltype(R)::value;
+        if (r == rc) fd_box_face<L, SF, rc>(p, nb, sg, q1, a1, qp, ap, fMJ, MJIn, sf);
+      });
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) sx[((2 * r + 1) * Ns + s) * Np + ijk] = sf[s];
+    }
+  }
+  __syncthreads();
+  if (!active || rg > 0) return;
+  double acc[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) {
+    acc[s] = ep.start(s, sx[s * Np + ijk]);
+#pragma unroll
+    for (int d = 1; d < D; ++d) acc[s] = acc[s] + sx[(2 * d * Ns + s) * Np + ijk];
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (idx[d] == 0 || idx[d] == NQ - 1) acc[s] -= sx[((2 * d + 1) * Ns + s) * Np + ijk];
+  }
+  ep.store(p, node, q1, acc);
+}
+
 // Largest workgroup of the form with a thread per node and direction: the 2-D kernels' (every shape fits).
 // Per stage, one thread per node against one per node and direction: vortex 8^2 N = 4 12.2 -> 8.2 us,
 // 32^2 N = 3 8.8 -> 6.8, 30^2 N = 7 14.1 -> 12.6, 64^2 N = 4 13.5 -> 13.5, 45^2 N = 6 16.9 -> 16.4.  In 3-D its
@@ -442,6 +593,27 @@ fd_box_dirs_kernel_batch(const BatchEntry* __restrict__ tab, int n, int parity, 
                               tab[i].buf[1 - parity], b * tab[i].dt, epw);
 }
 
+template <class L, int NQ, int SF>
+__global__ void __launch_bounds__(FD_PAIRS_THREADS)
+    fd_box_pairs_kernel(const DevDG p, const double* __restrict__ q, double* __restrict__ dq, double alpha, int assign,
+                        double* __restrict__ qout, double bdt, int epw, int group) {
+  extern __shared__ double lds[];
+  StageEnd<L> ep(dq, alpha, assign, qout, bdt);
+  fd_box_pairs_node<L, NQ, SF>(p, lds, xcd_block(), q, ep, epw, group);
+}
+
+// Whether a mesh's pairs are dealt out over groups of threads: where every CU has one workgroup at most.  Per
+// pass of two LSRK54 steps, against a thread per node and direction (2-D) or per node (3-D), with up to 256
+// workgroups: vortex 8^2 N = 4 78 -> 66 us, 16^2 N = 4 74 -> 66, 16^2 N = 7 96 -> 75, 32^2 N = 3 63 -> 60,
+// bubble 6^3 N = 4 146 -> 113, 5^3 N = 3 120 -> 91, 12^3 N = 1 87 -> 69; with more: vortex 24^2 N = 4 83 -> 97,
+// 20^2 N = 6 103 -> 113, bubble 7^3 N = 4 208 -> 206, 7^3 N = 3 125 -> 163.
+constexpr int FD_PAIRS_BLOCKS = 256;
+template <class L, int NQ>
+bool fd_box_pairs(const DevDG& p, int blocks, int threads) {
+  using S = FdPairs<L, NQ>;
+  return blocks <= FD_PAIRS_BLOCKS && S::groups(threads) > 1 && S::lds(p.epw) <= 160 * 1024;
+}
+
 ATM_KERNEL_PAIR(fd_box_kernel, fd_box_body, class L ATM_COMMA int NQ ATM_COMMA int SF, L ATM_COMMA NQ ATM_COMMA SF)
 
 template <class L, int NQ, int SF>
@@ -451,6 +623,13 @@ hipError_t launch_fd_box(const DevDG& p, hipStream_t st, const double* q, double
   if (p.epw < 1 || threads > 512) return hipErrorInvalidConfiguration;
   const int blocks = (p.K + p.epw - 1) / p.epw;
   if (blocks == 0) return hipSuccess;
+  if constexpr (L::D > 1)
+    if (fd_box_pairs<L, NQ>(p, blocks, threads)) {
+      using S = FdPairs<L, NQ>;
+      hipLaunchKernelGGL((fd_box_pairs_kernel<L, NQ, SF>), dim3(blocks), dim3(L::D * S::groups(threads) * threads),
+                         S::lds(p.epw), st, p, q, dq, alpha, assign, qout, bdt, p.epw, threads);
+      return hipGetLastError();
+    }
   if constexpr (fd_box_dirs_threads<L>() > 0)
     if (L::D * threads <= fd_box_dirs_threads<L>()) {
       hipLaunchKernelGGL((fd_box_dirs_kernel<L, NQ, SF>), dim3(blocks), dim3(L::D * threads), p.lds, st, p, q, dq,

@@ -139,6 +139,36 @@ def test_reference_order_box_kernels_against_the_general_ones(law, dim, Kd, kw, 
     assert np.abs(a - b).max() <= 2e-12 * np.abs(b).max()
 
 
+# 2-D elements of N = 7 and 3-D ones of N = 3 take a workgroup each: 256 of them, and one more
+DEALT = FAST + [("euler", 2, (16, 16), {}), ("euler", 2, (257, 1), {}),
+                ("euler_gravity", 3, (8, 8, 4), dict(bc="reflect", periodic=False)),
+                ("euler_gravity", 3, (257, 1, 1), dict(bc="reflect", periodic=False))]
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("sflux", ["roe", "rusanov"])
+@pytest.mark.parametrize("law,dim,Kd,kw", DEALT, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(DEALT)])
+def test_reference_order_pairs_dealt_out_over_threads(law, dim, Kd, kw, sflux, N):
+    """A small mesh's kernel, which deals a line's pairs out, in one-, two- and three-element workgroups against
+    the batched one, which does not: the same operations in the same order, so the same bits."""
+    import atum_hip as A
+    box, _, q0 = pair(law, dim, N, Kd, form="ec", sflux=sflux, seed=30 + N, **kw)
+    q = box.fieldarray(q0)
+    A.LSRKEnsemble([box], [q], [1e-4]).run(2)
+    box.ctx.sync()
+    want = q.numpy()
+    assert np.isfinite(want).all() and np.abs(want - q0).max() > 0
+    default = box.epw
+    for epw in (default, 1, 2, 3):
+        if epw != default and epw not in box.epw_candidates():
+            continue
+        box.epw = epw
+        q = box.fieldarray(q0)
+        A.LSRK54(box, q, 1e-4).run(q, 2)
+        box.ctx.sync()
+        np.testing.assert_array_equal(q.numpy(), want)
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("sflux", ["roe", "rusanov"])
 @pytest.mark.parametrize("law,dim,Kd,kw", FAST, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(FAST)])
