@@ -102,7 +102,11 @@ struct BoxEC {
       const double t = S * (sb * rl * (Pa[D + 2] - Pb[D + 2]));
       *ta = t * Pa[D + 3];
       *tb = t * Pb[D + 3];
+      asm("" : "+v"(*ta));
     }
+    // rounded here: a kernel could otherwise fuse the last product of one into the sum it goes to and another not
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) asm("" : "+v"(sf[s]));
   }
 };
 
@@ -424,6 +428,154 @@ ATM_DEV void fast_box_node(const DevDG& p, double* lds, int64_t blk, const doubl
   ep.store(p, node, q1, acc);
 }
 
+// An element's work dealt out by role: group 0 of a workgroup's threads takes direction 0 and the update, group
+// r direction r, the last group the face fluxes.  The sums in the order of fast_box_node: same bits.
+template <class L, int NQ>
+struct FastRoles {
+  static constexpr bool GRAV = L::LAW == ATM_LAW_EULER_GRAVITY;
+  static constexpr int D = L::D, Ns = L::Ns, Np = ipow(NQ, D), M = NQ / 2, NPL = BoxEC<L>::NP;
+  // shares of one direction, [distance][s][node], half of the last distance's with even NQ
+  static constexpr int share = NQ % 2 == 0 ? (M - 1) * Ns * Np + Ns * (Np / 2) : M * Ns * Np;
+  // primitives, state and geopotential, shares, the later directions' sums, face fluxes
+  static constexpr int state = NPL * Np, xch = state + (Ns + GRAV) * Np, sum = xch + D * share,
+                       faces = sum + (D - 1) * Ns * Np, stride = faces + 2 * D * (Np / NQ) * Ns;
+  static constexpr size_t lds(int epw) { return sizeof(double) * (size_t)(NQ * NQ + NQ + epw * stride); }
+};
+
+template <class L, int NQ, int SF, class EP>
+ATM_DEV void fast_box_roles_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep,
+                                 int epw) {
+#pragma clang fp contract(fast)
+  using EC = BoxEC<L>;
+  using S = FastRoles<L, NQ>;
+  using BF = BoxFaces<L, SF, NQ>;
+  constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = S::Np, M = S::M, NPL = S::NPL;
+  constexpr bool HALF = NQ % 2 == 0, GRAV = S::GRAV;
+  double* sS = lds;             // S_ab / 2 at [b + NQ a]
+  double* siw = lds + NQ * NQ;  // 1 / w_a
+  const int group = blockDim.x / (D + 1);
+  const int role = __builtin_amdgcn_readfirstlane(threadIdx.x / group);  // whole waves
+  const int tid = threadIdx.x - role * group;
+  const int el = tid / Np;
+  const int ijk = tid - el * Np;
+  const uint32_t le = (uint32_t)blk * epw + el;  // position in the processing order
+  const bool active = el < epw && le < (uint32_t)p.K;
+  const uint32_t e = (p.sched && active) ? (uint32_t)p.sched[le] : le;
+  // a lane past the last element reads element 0 and writes nothing
+  double* sP = lds + NQ * NQ + NQ + (active ? el : 0) * S::stride;
+  const uint32_t e0 = active ? e : 0;
+  const uint32_t node = 8 * (e0 * Np + ijk);
+  const BoxElem<D>* rec = box_elem<D>(p, e0);
+  for (int t = threadIdx.x; t < NQ * NQ; t += blockDim.x) {
+    const int b = t % NQ, a = t / NQ;
+    sS[t] = 0.5 * (p.D[b + NQ * a] * p.bw[b] - p.D[a + NQ * b] * p.bw[a]);
+  }
+  for (int t = threadIdx.x; t < NQ; t += blockDim.x) siw[t] = 1 / p.bw[t];
+  int idx[3];
+  node_index<D>(ijk, NQ, idx);
+  // a node of the upper half of its line in direction r, at line position c >= M, by its position there
+  auto half_pos = [&](int r, int c) {
+    int pos = 0, st = 1;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      pos += (d == r ? c - M : idx[d]) * st;
+      st *= d == r ? M : NQ;
+    }
+    return pos;
+  };
+  double q1[Ns], acc[Ns];
+  BF bf;
+  if (role == D) bf.load(rec, ijk);
+  if (role == 0) {
+    double a1[NA], P[NPL];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) q1[s] = ldo(p, q, s, node);
+    box_aux<L>(p, node, a1);
+    ep.load(p, node);
+    EC::prim(p.c, q1, GRAV ? a1[0] : 0.0, P);
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < NPL; ++k) sP[k * Np + ijk] = P[k];
+#pragma unroll
+      for (int s = 0; s < Ns; ++s) sP[S::state + s * Np + ijk] = q1[s];
+      if constexpr (GRAV) sP[S::state + Ns * Np + ijk] = a1[0];
+    }
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) acc[s] = 0.0;
+    if (active) L::sources(p.c, acc, q1, a1, all_dirs<L>(), false);
+  }
+  __syncthreads();  // tables, primitives and state written
+  double vol[Ns];
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) vol[s] = 0.0;
+  const double inv_gm1 = 1 / (p.c.gamma - 1);
+#pragma unroll
+  for (int m0 = 1; m0 <= M; m0 += BOX_SLOTS) {
+    for_dirs<0, D>([&](auto R) {
+      constexpr int r = decltype(R)::value, st = line_stride<NQ, r>();
+      if (role != r || !active) return;
+      const int a = idx[r], lbase = ijk - a * st;
+      double P1[NPL];
+#pragma unroll
+      for (int k = 0; k < NPL; ++k) P1[k] = sP[k * Np + ijk];
+#pragma unroll
+      for (int m = m0; m < m0 + BOX_SLOTS && m <= M; ++m) {
+        const bool hs = HALF && m == M;
+        if (hs && a >= M) continue;
+        const int b = a + m >= NQ ? a + m - NQ : a + m;
+        const int ib = lbase + b * st;
+        double P2[NPL], sf[Ns], ta, tb;
+#pragma unroll
+        for (int k = 0; k < NPL; ++k) P2[k] = sP[k * Np + ib];
+        EC::template pair<r>(inv_gm1, P1, P2, sS[b + NQ * a], sf, &ta, &tb);
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) vol[s] += sf[s];
+        if (GRAV) {
+          vol[1 + r] -= ta;
+          sf[1 + r] += tb;
+        }
+        // the partner's share, which it subtracts
+        double* slot = sP + S::xch + r * S::share + (m - 1) * Ns * Np + (hs ? half_pos(r, b) : ib);
+        const int xs = hs ? Np / 2 : Np;
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) slot[s * xs] = sf[s];
+      }
+    });
+    if (m0 == 1 && role == D && active) bf.run(p, rec, e, ijk, q, sP + S::faces, sP + S::state, siw[0]);
+    __syncthreads();  // the round's shares, and the face fluxes, written
+    for_dirs<0, D>([&](auto R) {
+      constexpr int r = decltype(R)::value;
+      if (role != r || !active) return;
+      const int a = idx[r];
+#pragma unroll
+      for (int m = m0; m < m0 + BOX_SLOTS && m <= M; ++m) {
+        const bool hs = HALF && m == M;
+        if (hs && a < M) continue;
+        const double* slot = sP + S::xch + r * S::share + (m - 1) * Ns * Np + (hs ? half_pos(r, a) : ijk);
+        const int xs = hs ? Np / 2 : Np;
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) vol[s] -= slot[s * xs];
+      }
+    });
+  }
+  if (active && role > 0 && role < D) {
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) sP[S::sum + ((role - 1) * Ns + s) * Np + ijk] = vol[s];
+  }
+  __syncthreads();  // the later directions' sums written
+  if (!active || role > 0) return;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const double gw = rec->g[d] * siw[idx[d]];
+#pragma unroll
+    for (int s = 0; s < Ns; ++s) acc[s] = fma(gw, d == 0 ? vol[s] : sP[S::sum + ((d - 1) * Ns + s) * Np + ijk], acc[s]);
+  }
+#pragma unroll
+  for (int s = 0; s < Ns; ++s) acc[s] = ep.start_fused(s, acc[s]);
+  BF::gather(idx, sP + S::faces, acc);
+  ep.store(p, node, q1, acc);
+}
+
 template <class L, int NQ, int SF>
 ATM_DEV void fast_box_body(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q,
                            double* __restrict__ dq, double alpha, int assign, double* __restrict__ qout, double bdt,
@@ -505,6 +657,32 @@ hipError_t launch_fast_box_multi_batch(const BatchEntry* tab, int n, int64_t blo
 }
 
 template <class L, int NQ, int SF>
+__global__ void __launch_bounds__(1024)
+    fast_box_roles_kernel(const DevDG p, const double* __restrict__ q, double* __restrict__ dq, double alpha,
+                          int assign, double* __restrict__ qout, double bdt, int epw) {
+  extern __shared__ double lds[];
+  StageEnd<L> ep(dq, alpha, assign, qout, bdt);
+  fast_box_roles_node<L, NQ, SF>(p, lds, xcd_block(), q, ep, epw);
+}
+
+// Whether a mesh's elements are dealt out by role: up to a wave per SIMD of the form with a thread per node
+// (six waves a CU in 2-D), which a node's chain of pairs bounds.  Per pass of two LSRK54 steps, a thread per node
+// against roles: vortex 8^2 N = 4 67 -> 50 us, 20^2 N = 6 77 -> 55, 36^2 N = 6 78 -> 67, 32^2 N = 7 77 -> 66,
+// 45^2 N = 4 60 -> 53, bubble 5^3 N = 4 83 -> 65, 8^3 N = 4 100 -> 77, 10^3 N = 3 84 -> 77, 6^3 N = 5 100 -> 86;
+// beyond: vortex 45^2 N = 6 85 -> 87, 70^2 N = 6 127 -> 152, bubble 10^3 N = 4 113 -> 129, 8^3 N = 5 126 -> 149.
+// 3-D elements of N = 1 gain nothing (10^3 63 -> 64), those of N = 6 and 7 have too many threads.
+template <class L, int NQ>
+constexpr bool fast_box_has_roles() {
+  return L::D == 2 || (NQ >= 3 && NQ <= 6);
+}
+template <class L, int NQ>
+bool fast_box_roles(const DevDG& p, int blocks, int threads) {
+  constexpr int waves = 256 * (L::D == 2 ? 6 : 4);
+  return (int64_t)blocks * threads <= 64 * waves && (L::D + 1) * threads <= 1024 &&
+         FastRoles<L, NQ>::lds(p.epw) <= 160 * 1024;
+}
+
+template <class L, int NQ, int SF>
 hipError_t launch_fast_box(const DevDG& p, hipStream_t st, const double* q, double* dq, double alpha, int assign,
                            double* qout, double bdt) {
   constexpr int Np = ipow(NQ, L::D);
@@ -512,6 +690,13 @@ hipError_t launch_fast_box(const DevDG& p, hipStream_t st, const double* q, doub
   if (p.epw < 1 || threads > fast_max_threads<L, NQ, SF>()) return hipErrorInvalidConfiguration;
   const int blocks = (p.K + p.epw - 1) / p.epw;
   if (blocks == 0) return hipSuccess;
+  if constexpr (fast_box_has_roles<L, NQ>())
+    if (fast_box_roles<L, NQ>(p, blocks, threads)) {
+      using S = FastRoles<L, NQ>;
+      hipLaunchKernelGGL((fast_box_roles_kernel<L, NQ, SF>), dim3(blocks), dim3((L::D + 1) * threads), S::lds(p.epw),
+                         st, p, q, dq, alpha, assign, qout, bdt, p.epw);
+      return hipGetLastError();
+    }
   hipLaunchKernelGGL((fast_box_kernel<L, NQ, SF>), dim3(blocks), dim3(threads), p.lds, st, p, q, dq, alpha, assign,
                      qout, bdt, p.epw);
   return hipGetLastError();

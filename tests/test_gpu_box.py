@@ -169,6 +169,36 @@ def test_reference_order_pairs_dealt_out_over_threads(law, dim, Kd, kw, sflux, N
         np.testing.assert_array_equal(q.numpy(), want)
 
 
+# N = 7 in 2-D and N = 3 in 3-D take a wave each: the most waves whose work is dealt out by role, and one more
+ROLES = FAST + [("euler", 2, (48, 32), {}), ("euler", 2, (1537, 1), {}),
+                ("euler_gravity", 3, (16, 8, 8), dict(bc="reflect", periodic=False)),
+                ("euler_gravity", 3, (1025, 1, 1), dict(bc="reflect", periodic=False))]
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("sflux", ["roe", "rusanov"])
+@pytest.mark.parametrize("law,dim,Kd,kw", ROLES, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(ROLES)])
+def test_fast_elements_dealt_out_by_role(law, dim, Kd, kw, sflux, N):
+    """A small mesh's kernel, which deals the directions and faces out, in one-, two- and three-element
+    workgroups against the batched one, which does not: the same operations in the same order, so the same bits."""
+    import atum_hip as A
+    box, _, q0 = pair(law, dim, N, Kd, form="ec", sflux=sflux, precision="fast", seed=40 + N, **kw)
+    q = box.fieldarray(q0)
+    A.LSRKEnsemble([box], [q], [1e-4]).run(2)
+    box.ctx.sync()
+    want = q.numpy()
+    assert np.isfinite(want).all() and np.abs(want - q0).max() > 0
+    default = box.epw
+    for epw in (default, 1, 2, 3):
+        if epw != default and epw not in box.epw_candidates():
+            continue
+        box.epw = epw
+        q = box.fieldarray(q0)
+        A.LSRK54(box, q, 1e-4).run(q, 2)
+        box.ctx.sync()
+        np.testing.assert_array_equal(q.numpy(), want)
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("sflux", ["roe", "rusanov"])
 @pytest.mark.parametrize("law,dim,Kd,kw", FAST, ids=[f"{c[0]}{c[1]}d{i}" for i, c in enumerate(FAST)])
