@@ -665,11 +665,12 @@ __global__ void __launch_bounds__(1024)
   fast_box_roles_node<L, NQ, SF>(p, lds, xcd_block(), q, ep, epw);
 }
 
-// Whether a mesh's elements are dealt out by role: up to a wave per SIMD of the form with a thread per node
-// (six waves a CU in 2-D), which a node's chain of pairs bounds.  Per pass of two LSRK54 steps, a thread per node
-// against roles: vortex 8^2 N = 4 67 -> 50 us, 20^2 N = 6 77 -> 55, 36^2 N = 6 78 -> 67, 32^2 N = 7 77 -> 66,
-// 45^2 N = 4 60 -> 53, bubble 5^3 N = 4 83 -> 65, 8^3 N = 4 100 -> 77, 10^3 N = 3 84 -> 77, 6^3 N = 5 100 -> 86;
-// beyond: vortex 45^2 N = 6 85 -> 87, 70^2 N = 6 127 -> 152, bubble 10^3 N = 4 113 -> 129, 8^3 N = 5 126 -> 149.
+// Whether a mesh's elements are dealt out by role: up to a wave per SIMD of the form with a thread per node and
+// two workgroups a CU (six waves a CU in 2-D), which a node's chain of pairs bounds.  Per pass of two LSRK54 steps,
+// a thread per node against roles: vortex 8^2 N = 4 67 -> 50 us, 20^2 N = 6 77 -> 57, 36^2 N = 6 79 -> 69,
+// 32^2 N = 7 77 -> 67, 45^2 N = 4 60 -> 54, bubble 5^3 N = 4 83 -> 64, 8^3 N = 4 100 -> 77, 8^3 N = 3 76 -> 62,
+// 6^3 N = 5 100 -> 78; beyond: vortex 45^2 N = 6 85 -> 87, 70^2 N = 6 127 -> 152, bubble 10^3 N = 3 84 -> 88,
+// 10^3 N = 4 113 -> 129, 8^3 N = 5 126 -> 149.
 // 3-D elements of N = 1 gain nothing (10^3 63 -> 64), those of N = 6 and 7 have too many threads.
 template <class L, int NQ>
 constexpr bool fast_box_has_roles() {
@@ -678,7 +679,7 @@ constexpr bool fast_box_has_roles() {
 template <class L, int NQ>
 bool fast_box_roles(const DevDG& p, int blocks, int threads) {
   constexpr int waves = 256 * (L::D == 2 ? 6 : 4);
-  return (int64_t)blocks * threads <= 64 * waves && (L::D + 1) * threads <= 1024 &&
+  return (L::D == 2 || blocks <= 512) && (int64_t)blocks * threads <= 64 * waves && (L::D + 1) * threads <= 1024 &&
          FastRoles<L, NQ>::lds(p.epw) <= 160 * 1024;
 }
 

@@ -139,10 +139,12 @@ def test_reference_order_box_kernels_against_the_general_ones(law, dim, Kd, kw, 
     assert np.abs(a - b).max() <= 2e-12 * np.abs(b).max()
 
 
-# 2-D elements of N = 7 and 3-D ones of N = 3 take a workgroup each: 256 of them, and one more
+# 2-D elements of N = 7 and 3-D ones of N = 3 take a workgroup each: 256 of them, and one more; 512, and one more
 DEALT = FAST + [("euler", 2, (16, 16), {}), ("euler", 2, (257, 1), {}),
                 ("euler_gravity", 3, (8, 8, 4), dict(bc="reflect", periodic=False)),
-                ("euler_gravity", 3, (257, 1, 1), dict(bc="reflect", periodic=False))]
+                ("euler_gravity", 3, (257, 1, 1), dict(bc="reflect", periodic=False)),
+                ("euler_gravity", 3, (8, 8, 8), dict(bc="reflect", periodic=False)),
+                ("euler_gravity", 3, (513, 1, 1), dict(bc="reflect", periodic=False))]
 
 
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 7])
@@ -169,10 +171,10 @@ def test_reference_order_pairs_dealt_out_over_threads(law, dim, Kd, kw, sflux, N
         np.testing.assert_array_equal(q.numpy(), want)
 
 
-# N = 7 in 2-D and N = 3 in 3-D take a wave each: the most waves whose work is dealt out by role, and one more
+# N = 7 in 2-D and N = 3 in 3-D take a wave each: the most workgroups whose work is dealt out by role, and one more
 ROLES = FAST + [("euler", 2, (48, 32), {}), ("euler", 2, (1537, 1), {}),
-                ("euler_gravity", 3, (16, 8, 8), dict(bc="reflect", periodic=False)),
-                ("euler_gravity", 3, (1025, 1, 1), dict(bc="reflect", periodic=False))]
+                ("euler_gravity", 3, (8, 8, 8), dict(bc="reflect", periodic=False)),
+                ("euler_gravity", 3, (513, 1, 1), dict(bc="reflect", periodic=False))]
 
 
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7])
