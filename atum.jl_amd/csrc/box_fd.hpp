@@ -310,11 +310,6 @@ __global__ void __launch_bounds__(512)
   box_ark_pair<L, NQ, FdBoxBody<L, NQ, SF>>(p, pl, lds, q, a, epw);
 }
 
-template <class L, int NQ, int SF>
-hipError_t launch_fd_box_ark(const DevDG& p, const DevDG& pl, hipStream_t st, const double* q, const ArkSums& a) {
-  return launch_box_ark_pair<L, NQ>(fd_box_ark_kernel<L, NQ, SF>, 512, p, pl, st, q, a);
-}
-
 // One thread per node and direction: the waves of group r (blockDim / D threads) form direction r's volume
 // sum and face, and group 0 adds them up in the order above.  The same numbers; a node's chain of
 // pairs, which is all the time a small mesh takes, is D times shorter.
@@ -411,13 +406,14 @@ constexpr int FD_PAIRS_THREADS = 768;
 
 // The pairs of a line dealt out too: group (r, g) forms direction r's pairs with the partners n = g, g + G, ...
 // and leaves their fluxes in LDS; group (r, 0) then adds them up in the order of fd_box_dir while the last one,
-// (r, G - 1), forms the face, and group (0, 0) puts the directions together.  The same numbers.  A small mesh
+// (r, G - 1), forms the face, and group (0, 0) puts the directions together.  The same numbers.  Without DEAL
+// there is one group a direction, which adds its pairs up as it forms them.  A small mesh
 // is bound by one node's chain of pairs (128 waves, bubble 4^3 N = 4, take 14 us a stage, 9 cycles an
 // instruction), which this makes G times shorter.
-template <class L, int NQ>
+template <class L, int NQ, bool DEAL>
 struct FdPairs {
   static constexpr int D = L::D, Ns = L::Ns, Np = ipow(NQ, D), NP = BoxPairEC<L>::NP;
-  static constexpr int NF = D * NQ * Ns;  // flux planes, [r][n][s]
+  static constexpr int NF = DEAL ? D * NQ * Ns : 0;  // flux planes, [r][n][s]
   // planes: primitives, MJ, fluxes, then [r][volume, face][s]
   static constexpr int stride = (NP + 1 + NF + 2 * D * Ns) * Np;
   // groups of partners for workgroups of `threads` per group (1: none)
@@ -428,15 +424,15 @@ struct FdPairs {
   static constexpr size_t lds(int epw) { return sizeof(double) * (size_t)(NQ * NQ + NQ + epw * stride); }
 };
 
-template <class L, int NQ, int SF, class EP>
+template <class L, int NQ, int SF, bool DEAL, class EP>
 ATM_DEV void fd_box_pairs_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw,
                                int group) {
   using PF = BoxPairEC<L>;
-  using S = FdPairs<L, NQ>;
+  using S = FdPairs<L, NQ, DEAL>;
   constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = S::Np, NP = S::NP;
   double* sD = lds;
   double* sw = lds + NQ * NQ;
-  const int G = blockDim.x / (D * group);
+  const int G = DEAL ? blockDim.x / (D * group) : 1;
   const int rg = __builtin_amdgcn_readfirstlane(threadIdx.x / group);  // whole waves
   const int r = rg / G, gr = rg - r * G;
   const int tid = threadIdx.x - rg * group;
@@ -490,6 +486,13 @@ ATM_DEV void fd_box_pairs_node(const DevDG& p, double* lds, int64_t blk, const d
     for_dirs<0, D>([&](auto R) {
       constexpr int rc = decltype(R)::value, st = line_stride<NQ, rc>();
       if (r != rc) return;
+      if constexpr (!DEAL) {
+        double dl[Ns];
+        fd_box_dir<L, NQ, rc>(p, sD, sP, ijk, ir, g, MJn, MJIn, q1, a1, P1, dl);
+#pragma unroll
+        for (int s = 0; s < Ns; ++s) sx[(2 * rc * Ns + s) * Np + ijk] = dl[s];
+        return;
+      }
       const double* line = sP + ijk - ir * st;
 #pragma unroll 1
       for (int n = gr; n < NQ; n += G) {
@@ -502,9 +505,9 @@ ATM_DEV void fd_box_pairs_node(const DevDG& p, double* lds, int64_t blk, const d
       }
     });
   }
-  __syncthreads();  // fluxes written
+  if (DEAL) __syncthreads();  // fluxes written
   if (active) {
-    if (gr == 0) {
+    if (DEAL && gr == 0) {
       double dl[Ns];
 #pragma unroll
       for (int s = 0; s < Ns; ++s) dl[s] = -0.0;
@@ -559,9 +562,9 @@ ATM_DEV void fd_box_pairs_node(const DevDG& p, double* lds, int64_t blk, const d
 
 // Largest workgroup of the form with a thread per node and direction: the 2-D kernels' (every shape fits).
 // Per stage, one thread per node against one per node and direction: vortex 8^2 N = 4 12.2 -> 8.2 us,
-// 32^2 N = 3 8.8 -> 6.8, 30^2 N = 7 14.1 -> 12.6, 64^2 N = 4 13.5 -> 13.5, 45^2 N = 6 16.9 -> 16.4.  In 3-D its
-// six-wave workgroups of 168 registers leave too few of them resident: bubble 12^3 N = 4 38 -> 57 us, 14^3
-// N = 3 26.4 -> 30.4.
+// 32^2 N = 3 8.8 -> 6.8, 30^2 N = 7 14.1 -> 12.6, 64^2 N = 4 13.5 -> 13.5, 45^2 N = 6 16.9 -> 16.4.  Of a larger
+// 3-D mesh its six-wave workgroups of 168 registers leave too few resident: bubble 12^3 N = 4 38 -> 57 us,
+// 14^3 N = 3 26.4 -> 30.4.
 template <class L>
 constexpr int fd_box_dirs_threads() {
   return L::D == 2 ? 1024 : 0;
@@ -593,13 +596,13 @@ fd_box_dirs_kernel_batch(const BatchEntry* __restrict__ tab, int n, int parity, 
                               tab[i].buf[1 - parity], b * tab[i].dt, epw);
 }
 
-template <class L, int NQ, int SF>
+template <class L, int NQ, int SF, bool DEAL>
 __global__ void __launch_bounds__(FD_PAIRS_THREADS)
     fd_box_pairs_kernel(const DevDG p, const double* __restrict__ q, double* __restrict__ dq, double alpha, int assign,
                         double* __restrict__ qout, double bdt, int epw, int group) {
   extern __shared__ double lds[];
   StageEnd<L> ep(dq, alpha, assign, qout, bdt);
-  fd_box_pairs_node<L, NQ, SF>(p, lds, xcd_block(), q, ep, epw, group);
+  fd_box_pairs_node<L, NQ, SF, DEAL>(p, lds, xcd_block(), q, ep, epw, group);
 }
 
 // Whether a mesh's pairs are dealt out over groups of threads: where every CU has one workgroup at most.  Per
@@ -608,10 +611,58 @@ __global__ void __launch_bounds__(FD_PAIRS_THREADS)
 // bubble 6^3 N = 4 146 -> 113, 5^3 N = 3 120 -> 91, 12^3 N = 1 87 -> 69; with more: vortex 24^2 N = 4 83 -> 97,
 // 20^2 N = 6 103 -> 113, bubble 7^3 N = 4 208 -> 206, 7^3 N = 3 125 -> 163.
 constexpr int FD_PAIRS_BLOCKS = 256;
-template <class L, int NQ>
-bool fd_box_pairs(const DevDG& p, int blocks, int threads) {
-  using S = FdPairs<L, NQ>;
-  return blocks <= FD_PAIRS_BLOCKS && S::groups(threads) > 1 && S::lds(p.epw) <= 160 * 1024;
+// In 3-D up to two workgroups a CU and a wave per SIMD the directions alone are dealt out.  Per pass, a thread per
+// node against one per node and direction: bubble 7^3 N = 3 123 -> 100 us, 8^3 N = 4 207 -> 189, 9^3 N = 2
+// 114 -> 94, 6^3 N = 5 166 -> 156, 14^3 N = 1 93 -> 79, two ARK23 steps on 8x8x6 N = 3 137 -> 123; beyond:
+// 10^3 N = 3 132 -> 131, 12^3 N = 2 121 -> 122, 20^3 N = 1 102 -> 105, 11x11x7 157 -> 156.
+constexpr int FD_DIRS_BLOCKS = 512, FD_DIRS_WAVES = 1024;
+// Calls f(DEAL, groups of partners, LDS) if a launch takes that form
+template <class L, int NQ, class F>
+bool fd_box_dealt(const DevDG& p, int blocks, int threads, F&& f) {
+  if (p.epw < 1 || blocks < 1) return false;
+  const int G = FdPairs<L, NQ, true>::groups(threads);
+  const size_t lds = FdPairs<L, NQ, true>::lds(p.epw);
+  if (blocks <= FD_PAIRS_BLOCKS && G > 1 && lds <= 160 * 1024) {
+    f(std::true_type{}, G, lds);
+    return true;
+  }
+  if constexpr (L::D == 3) {
+    const size_t lds1 = FdPairs<L, NQ, false>::lds(p.epw);
+    if (L::D * threads <= FD_PAIRS_THREADS && blocks <= FD_DIRS_BLOCKS &&
+        (int64_t)blocks * threads <= 64 * FD_DIRS_WAVES && lds1 <= 160 * 1024) {
+      f(std::false_type{}, 1, lds1);
+      return true;
+    }
+  }
+  return false;
+}
+
+template <class L, int NQ, int SF, bool DEAL>
+struct FdPairsBody {
+  template <class EP>
+  ATM_DEV static void run(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
+    fd_box_pairs_node<L, NQ, SF, DEAL>(p, lds, blk, q, ep, epw, (epw * ipow(NQ, L::D) + 63) / 64 * 64);
+  }
+};
+
+template <class L, int NQ, int SF, bool DEAL>
+__global__ void __launch_bounds__(FD_PAIRS_THREADS)
+    fd_box_pairs_ark_kernel(const DevDG p, const DevDG pl, const double* __restrict__ q, const ArkSums a, int epw) {
+  extern __shared__ double lds[];
+  box_ark_pair<L, NQ, FdPairsBody<L, NQ, SF, DEAL>>(p, pl, lds, q, a, epw);
+}
+
+template <class L, int NQ, int SF>
+hipError_t launch_fd_box_ark(const DevDG& p, const DevDG& pl, hipStream_t st, const double* q, const ArkSums& a) {
+  const int threads = ((p.epw * p.Np + 63) / 64) * 64, blocks = p.epw < 1 ? 0 : (p.K + p.epw - 1) / p.epw;
+  // (an element's planes of the explicit form outnumber the implicit one's)
+  if (fd_box_dealt<L, NQ>(p, blocks, threads, [&](auto deal, int G, size_t lds) {
+        constexpr bool DEAL = decltype(deal)::value;
+        hipLaunchKernelGGL((fd_box_pairs_ark_kernel<L, NQ, SF, DEAL>), dim3(blocks), dim3(L::D * G * threads), lds, st, p,
+                           pl, q, a, p.epw);
+      }))
+    return hipGetLastError();
+  return launch_box_ark_pair<L, NQ>(fd_box_ark_kernel<L, NQ, SF>, 512, p, pl, st, q, a);
 }
 
 ATM_KERNEL_PAIR(fd_box_kernel, fd_box_body, class L ATM_COMMA int NQ ATM_COMMA int SF, L ATM_COMMA NQ ATM_COMMA SF)
@@ -624,12 +675,12 @@ hipError_t launch_fd_box(const DevDG& p, hipStream_t st, const double* q, double
   const int blocks = (p.K + p.epw - 1) / p.epw;
   if (blocks == 0) return hipSuccess;
   if constexpr (L::D > 1)
-    if (fd_box_pairs<L, NQ>(p, blocks, threads)) {
-      using S = FdPairs<L, NQ>;
-      hipLaunchKernelGGL((fd_box_pairs_kernel<L, NQ, SF>), dim3(blocks), dim3(L::D * S::groups(threads) * threads),
-                         S::lds(p.epw), st, p, q, dq, alpha, assign, qout, bdt, p.epw, threads);
+    if (fd_box_dealt<L, NQ>(p, blocks, threads, [&](auto deal, int G, size_t lds) {
+          constexpr bool DEAL = decltype(deal)::value;
+          hipLaunchKernelGGL((fd_box_pairs_kernel<L, NQ, SF, DEAL>), dim3(blocks), dim3(L::D * G * threads), lds, st, p,
+                             q, dq, alpha, assign, qout, bdt, p.epw, threads);
+        }))
       return hipGetLastError();
-    }
   if constexpr (fd_box_dirs_threads<L>() > 0)
     if (L::D * threads <= fd_box_dirs_threads<L>()) {
       hipLaunchKernelGGL((fd_box_dirs_kernel<L, NQ, SF>), dim3(blocks), dim3(L::D * threads), p.lds, st, p, q, dq,
