@@ -161,10 +161,8 @@ std::vector<double> box_tables(int dim, int Nq, const double* w) {
   return tab;
 }
 
-size_t box_elem_bytes(int dim) { return (size_t)(2 * dim + 1) * sizeof(double) + (size_t)2 * dim * sizeof(int32_t); }
-
 bool box_kernels(const atm_dg* dg, const atm_dg_desc* d, Resolved* r) {
-  if (dg->dev.K < 1 || dg->Ns * dg->Ntot >= BOX_MAX_STATE) return false;
+  if (dg->dev.K < 1 || !box_fits(dg->dim, dg->Np, dg->Ns, dg->dev.K)) return false;
   *r = resolve_box(d, dg->Nq);
   return r->fn && r->lds <= dg->ctx->max_lds;
 }
@@ -263,3 +261,8 @@ Resolved resolve_box(const atm_dg_desc* d, int Nq) {
 }
 
 }  // namespace atm
+
+extern "C" int atm_box_elements_fit(int dim, int N, int Ns, int64_t K) {
+  if (dim < 1 || dim > 3 || N < 1 || N > 7 || Ns < 1 || K < 0) return ATM_ERR_ARG;
+  return atm::box_fits(dim, atm::ipow(N + 1, dim), Ns, K) ? 1 : 0;
+}

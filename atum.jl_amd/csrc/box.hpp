@@ -28,10 +28,20 @@ struct BoxElem {
   int32_t nb[2 * D];  // neighbour element of each face, or minus the boundary tag
 };
 
-// The box kernels address fields with 32-bit byte offsets from a uniform base (a scalar register and
-// one vector register per address instead of 64-bit vector arithmetic for every load), so they take
-// operators whose state is below 4 GB; larger ones run the general kernels.
-constexpr int64_t BOX_MAX_STATE = (int64_t)1 << 29;  // doubles
+// The box kernels address fields and records with 32-bit byte offsets from a uniform base (a scalar register and
+// one vector register per address instead of 64-bit vector arithmetic for every load), so they take operators
+// whose state is below 4 GB and whose records end there (one component at N = 1, in 1-D also N = 2, has larger
+// records than states); larger ones run the general kernels.  Np: nodes of an element, Ns: components.
+constexpr int64_t BOX_MAX_STATE = (int64_t)1 << 29;    // doubles
+constexpr int64_t BOX_MAX_RECORDS = (int64_t)1 << 32;  // bytes
+constexpr size_t box_elem_bytes(int dim) {
+  return (size_t)(2 * dim + 1) * sizeof(double) + (size_t)2 * dim * sizeof(int32_t);
+}
+static_assert(sizeof(BoxElem<1>) == box_elem_bytes(1) && sizeof(BoxElem<2>) == box_elem_bytes(2) &&
+              sizeof(BoxElem<3>) == box_elem_bytes(3));
+constexpr bool box_fits(int dim, int64_t Np, int64_t Ns, int64_t K) {
+  return K < BOX_MAX_STATE && Ns * Np * K < BOX_MAX_STATE && K * (int64_t)box_elem_bytes(dim) <= BOX_MAX_RECORDS;
+}
 
 // A global pointer kept in scalar registers: the empty statement hides it from the address arithmetic
 // of the lanes, so that a load takes it as the base and the lane's offset as one register.

@@ -99,10 +99,9 @@ Resolved resolve_box(const atm_dg_desc* d, int Nq);
 int dg_box(atm_dg* dg, const atm_dg_desc* d);
 
 // The parts of it for an operator that is known to consist of boxes: whether there are kernels, the
-// weight tables from the LGL weights, a record's size, and the selection.
+// weight tables from the LGL weights, and the selection.
 bool box_kernels(const atm_dg* dg, const atm_dg_desc* d, Resolved* r);
 std::vector<double> box_tables(int dim, int Nq, const double* w);
-size_t box_elem_bytes(int dim);
 void dg_use_box(atm_dg* dg, const Resolved& r, const void* rec, const double* tab);
 
 // The linear operator a banded factorisation was built from.

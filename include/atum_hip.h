@@ -200,6 +200,11 @@ int64_t atm_dg_nnodes(const atm_dg* dg);
  * schedule buffers), as the serving scheduler counts it against its budget.  No
  * counterpart in the reference. */
 int64_t atm_dg_device_bytes(const atm_dg* dg);
+/* 1 if an operator of K axis-aligned box elements of dim directions, degree N and Ns
+ * components is within the range of the kernels on the compact box geometry (32-bit
+ * offsets: state and per-element records below 4 GB each), 0 if it runs the general
+ * kernels.  Arithmetic only, no device.  No counterpart in the reference. */
+int atm_box_elements_fit(int dim, int N, int Ns, int64_t K);
 
 /* The rhs! protocol: replaces `(dg::DGSEM)(dq, q, time; increment)`
  * (src/dgsem.jl:59-98).  increment != 0: dq += L(q); else dq = L(q).
