@@ -28,10 +28,11 @@ __device__ double candidate(double x, int c) {
 // the candidate to keep: the quotient itself if it fits, else any that does
 __device__ int pick(unsigned mask) { return (mask >> (CAND / 2)) & 1u ? CAND / 2 : __ffs(mask) - 1; }
 
-// One workgroup per element: writes its record, or sets *bad when its arrays are not those of a box.
+// One workgroup per element: writes its record, or sets *bad when its arrays are not those of a box.  lift: the
+// kernels scale what a face adds by g_r / w_end in place of faceMJ MJI, so the face Jacobians have to be J g_r.
 __global__ void __launch_bounds__(256)
     box_detect_kernel(DevDG p, int dim, const double* __restrict__ wp, const double* __restrict__ wf, char* rec,
-                      int bytes, int32_t* bad) {
+                      int bytes, int lift, int32_t* bad) {
   __shared__ unsigned mJ, mF[3];
   __shared__ int ok;
   for (int64_t e = blockIdx.x; e < p.K; e += gridDim.x) {
@@ -99,11 +100,16 @@ __global__ void __launch_bounds__(256)
           g[r] = p.g[(int64_t)(r + dim * r) * p.Ntot + e * p.Np];
           fJ[r] = candidate(fJ0[r], pick(mF[r]));
         }
+        const double J = candidate(J0, pick(mJ));
+        // (a box's own are a few roundings apart)
+        if (lift)
+          for (int r = 0; r < dim; ++r)
+            if (!(fabs(g[r] * J - fJ[r]) <= 64 * 2.220446049250313e-16 * fJ[r])) *bad = 1;
         for (int f = 0; f < 2 * dim; ++f) {
           const int tag = p.bctag[e * (2 * dim) + f];
           nb[f] = tag ? -tag : (int32_t)(p.faceix_p[e * p.Nfp + f * p.Nfpf] / p.Np);
         }
-        store_record(rec + e * bytes, dim, g, candidate(J0, pick(mJ)), fJ, nb);
+        store_record(rec + e * bytes, dim, g, J, fJ, nb);
       } else {
         *bad = 1;
       }
@@ -185,6 +191,11 @@ void dg_use_box(atm_dg* dg, const Resolved& r, const void* rec, const double* ta
   p.lds = (int)r.lds;
 }
 
+// whether the operator's kernels are FAST ones, which read neither Jacobians nor face Jacobians
+static int box_lift(const atm_dg_desc* d) {
+  return d->volume_form == ATM_FORM_FLUX_DIFFERENCING && d->precision == ATM_PRECISION_FAST;
+}
+
 int dg_box(atm_dg* dg, const atm_dg_desc* d) {
   DevDG& p = dg->dev;
   Resolved r;
@@ -207,7 +218,7 @@ int dg_box(atm_dg* dg, const atm_dg_desc* d) {
   hipError_t e = hipMemcpy(mem, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(box_detect_kernel, dim3(p.K < 65536 ? p.K : 65536), dim3(Np > 128 ? 256 : 64), 0, s, p, dim,
-                       dtab + Nq, dtab + Nq + Np, rec, (int)bytes, bad);
+                       dtab + Nq, dtab + Nq + Np, rec, (int)bytes, box_lift(d), bad);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s);

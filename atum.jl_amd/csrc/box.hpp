@@ -8,9 +8,11 @@
 // 56 bytes per element of 16 nodes instead of 1280 (the state, dq and the new state are 2048).
 //
 // Whether an operator's elements are boxes is found from its geometry arrays when it is
-// created (box_detect): the values that the compact form reproduces have to equal the arrays
+// created (box_detect_kernel): the values that the compact form reproduces have to equal the arrays
 // bit for bit in every node and face point, so that both forms of a kernel compute with the
-// same numbers.  Operators with any other element keep the general kernels.
+// same numbers; for the FAST kernels, which use 2/h for faceMJ MJI too (box_fast.hpp), the face
+// Jacobians also have to be the Jacobian times 2/h.  Operators with any other element keep the
+// general kernels.
 #pragma once
 #include <algorithm>
 #include <type_traits>
