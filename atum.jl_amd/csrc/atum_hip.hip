@@ -1460,16 +1460,7 @@ int atm_dg_create(atm_ctx* ctx, const atm_dg_desc* d, atm_dg** out) {
   atm_dg* dg = nullptr;
   int rc = dg_prepare(ctx, d, &dg);
   if (rc) return rc;
-  DevDG& p = dg->dev;
-  const size_t dd = (size_t)d->dim * d->dim;
-  if ((rc = upload_copy(dg, d->D, (size_t)Nq * Nq, &p.D)) ||
-      (rc = upload_copy(dg, d->g, dd * Ntot, &p.g)) ||
-      (rc = upload_copy(dg, d->MJ, (size_t)Ntot, &p.MJ)) ||
-      (rc = upload_copy(dg, d->MJI, (size_t)Ntot, &p.MJI)) ||
-      (rc = upload_copy(dg, d->faceMJ, (size_t)NF, &p.faceMJ)) ||
-      (rc = upload_copy(dg, d->normal, (size_t)d->dim * NF, &p.normal)) ||
-      (rc = upload_copy(dg, d->faceix_p, (size_t)NF, &p.faceix_p)) ||
-      (rc = upload_copy(dg, d->bctag, (size_t)2 * d->dim * d->K, &p.bctag)) || (rc = dg_box(dg, d))) {
+  if ((rc = dg_upload_geometry(dg, d))) {
     atm_dg_destroy(dg);
     return rc;
   }

@@ -94,9 +94,9 @@ int dg_prepare(atm_ctx* ctx, const atm_dg_desc* d, atm_dg** out);
 // The kernels for an operator whose elements are all boxes (box.hpp); fn == nullptr if none.
 Resolved resolve_box(const atm_dg_desc* d, int Nq);
 
-// Looks whether the operator's elements are all boxes, its geometry arrays being on the device;
-// if so, and there are kernels for it, builds the compact geometry and selects them.
-int dg_box(atm_dg* dg, const atm_dg_desc* d);
+// Uploads the geometry arrays (checked by the caller).  Where there are box kernels for the operator and its
+// elements are all boxes, builds the compact geometry and selects them.
+int dg_upload_geometry(atm_dg* dg, const atm_dg_desc* d);
 
 // The parts of it for an operator that is known to consist of boxes: whether there are kernels, the
 // weight tables from the LGL weights, and the selection.
