@@ -91,6 +91,7 @@ _sig("atm_dg_nstates", c_int, [c_void_p])
 _sig("atm_dg_nnodes", c_int64, [c_void_p])
 _sig("atm_dg_device_bytes", c_int64, [c_void_p])
 _sig("atm_box_elements_fit", c_int, [c_int, c_int, c_int, c_int64])
+_sig("atm_dg_box_elements", c_int, [c_void_p])
 _sig("atm_dg_get_epw", c_int, [c_void_p])
 _sig("atm_dg_set_schedule", c_int, [c_void_p, ctypes.POINTER(ctypes.c_int32), c_int64])
 _sig("atm_dg_set_epw", c_int, [c_void_p, c_int])

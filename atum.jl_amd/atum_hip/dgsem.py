@@ -108,9 +108,6 @@ class DGSEM:
         d.naux = naux
         d.precision = _lib.PRECISION_IDS[precision]
         self.precision = precision
-        # what selects the element kernel (with K, the key of the workgroup-shape tuning)
-        self.kernel_key = (law.law, dim, grid.N, d.volume_form, d.volume_flux, d.surface_flux, d.dirmask,
-                           precision, d.fd_kernel)
         d.gamma = float(getattr(law, "gamma", 1.4))
         d.grav = float(getattr(law, "grav", 9.81))
         d.omega = float(prob.omega)
@@ -151,6 +148,9 @@ class DGSEM:
             self.ctx.check(_lib.lib.atm_dg_create(self.ctx.h, ctypes.byref(d), ctypes.byref(h)),
                            "atm_dg_create")
         self.h = h
+        # what selects the element kernel (with K, the key of the workgroup-shape tuning)
+        self.kernel_key = (law.law, dim, grid.N, d.volume_form, d.volume_flux, d.surface_flux, d.dirmask,
+                           precision, d.fd_kernel) + (("box",) if _lib.lib.atm_dg_box_elements(h) else ())
         self.Ns = _lib.lib.atm_dg_nstates(h)
         self.element_order = element_order
         if element_order == "morton" and grid.K > 1:

@@ -329,3 +329,5 @@ extern "C" int atm_box_elements_fit(int dim, int N, int Ns, int64_t K) {
   if (dim < 1 || dim > 3 || N < 1 || N > 7 || Ns < 1 || K < 0) return ATM_ERR_ARG;
   return atm::box_fits(dim, atm::ipow(N + 1, dim), Ns, K) ? 1 : 0;
 }
+
+extern "C" int atm_dg_box_elements(const atm_dg* dg) { return !dg ? ATM_ERR_ARG : dg->dev.box ? 1 : 0; }

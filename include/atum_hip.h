@@ -205,6 +205,10 @@ int64_t atm_dg_device_bytes(const atm_dg* dg);
  * offsets: state and per-element records below 4 GB each), 0 if it runs the general
  * kernels.  Arithmetic only, no device.  No counterpart in the reference. */
 int atm_box_elements_fit(int dim, int N, int Ns, int64_t K);
+/* 1 if the operator's elements were found to be axis-aligned boxes and its element
+ * kernels read the compact geometry, 0 if they are the general ones (the choice is part
+ * of what a workgroup shape is tuned for). */
+int atm_dg_box_elements(const atm_dg* dg);
 
 /* The rhs! protocol: replaces `(dg::DGSEM)(dq, q, time; increment)`
  * (src/dgsem.jl:59-98).  increment != 0: dq += L(q); else dq = L(q).
