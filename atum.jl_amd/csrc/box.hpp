@@ -247,6 +247,7 @@ ATM_DEV void box_surface_node(const DevDG& p, const BoxElem<L::D>& b, uint32_t e
 // EP: what a node's tendency goes into; load() is called with the node's other loads, store() last.
 template <class L, int NQ, int SF, int MASK, class EP>
 ATM_DEV void weak_box_node(const DevDG& p, double* lds, int64_t blk, const double* __restrict__ q, EP& ep, int epw) {
+  static_assert(SF == ATM_FLUX_RUSANOV, "box_surface_node is Rusanov's");
   constexpr int D = L::D, Ns = L::Ns, NA = L::NA, Np = ipow(NQ, D);
   double* sD = lds;
   double* sw = lds + NQ * NQ;

@@ -14,7 +14,7 @@ ATM_DEV double scalar(double c) {
   return c;
 }
 
-// f/atanh f and atanh(f)/f in u = f^2 <= LM_U0: Chebyshev interpolants of degree 6 (3e-19 off)
+// f/atanh f and atanh(f)/f in u = f^2 <= LM_U: Chebyshev interpolants of degree 6 (3e-19 off)
 ATM_DEV double lm_inverse(double u) {
 #pragma clang fp contract(fast)
   double s = u * -0.017268601586902934 + -0.02179015140718188;
