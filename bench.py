@@ -41,6 +41,19 @@ def algorithmic_bytes_per_stage(dim, Nq, K, Ns, naux):
     return per_elem * K
 
 
+def box_bytes_per_stage(dim, Nq, K, Ns, naux):
+    """Traffic that a stage cannot do without on axis-aligned box elements, whose kernels read no geometry array:
+    per node q and dq read+write (32*Ns) and aux (naux*8); per element one record of 2d+1 doubles and 2d int32."""
+    return K * (Nq ** dim * (32 * Ns + naux * 8) + (2 * dim + 1) * 8 + 2 * dim * 4)
+
+
+def stage_bytes(dg, naux):
+    """The bytes the operator's stage kernel has to move: its roofline fraction counts these."""
+    import atum_hip._lib as L
+    model = box_bytes_per_stage if L.lib.atm_dg_box_elements(dg.h) == 1 else algorithmic_bytes_per_stage
+    return model(dg.grid.dim, dg.grid.Nq, dg.grid.K, dg.Ns, naux)
+
+
 FP64_PEAK_TFS = 78.6  # MI355X FP64 (vector and matrix)
 
 
@@ -348,7 +361,7 @@ def weak_workload(args):
         raise SystemExit("bench: non-finite shallow-water state")
     dof = q0.size
     stages = 5 * args.steps
-    algo = algorithmic_bytes_per_stage(2, N + 1, grid.K, 4, 0)
+    algo = stage_bytes(dg, 0)
     kern_s = ms / 1e3 / stages
     achieved = algo / kern_s / 1e9
     return {"metric": "FP64 DOF-updates/s per RK stage (weak form, one instance)",
@@ -621,7 +634,7 @@ def main():
     dof = Ns * Np * K
     value = dof * stages / (ms / 1e3)
     naux = dg.auxstate.shape[0]
-    algo = algorithmic_bytes_per_stage(3, N + 1, K, Ns, naux)
+    algo = stage_bytes(dg, naux)
     kern_s = ms / 1e3 / stages
     achieved = algo / kern_s / 1e9
     # HBM bytes per launch come from rocprofv3 FETCH_SIZE / WRITE_SIZE counter runs of this
